@@ -1089,75 +1089,171 @@ void launch_tip_rms(const float* x, int C, const float* gamma, const float* beta
 }
 
 // ---------------------------------------------------------------------------------------------------------
-// Attention: one thread per query, keys and values staged 32 at a time in LDS, online softmax
+// Attention
 // ---------------------------------------------------------------------------------------------------------
 
-template <typename T, int D>
-__global__ __launch_bounds__(64) void attn_kernel(AttnArgs a) {
-  const int qi = blockIdx.x * 64 + threadIdx.x, h = blockIdx.y, n = blockIdx.z, tid = threadIdx.x;
-  const int kvh = h / (a.H / a.KV);
-  const bool in_range = qi < HW;
-  const int qrow = in_range ? qi : 0;
-  const T* qkv = (const T*)a.qkv;
-  float q[D], acc[D];
-  {
-    const T* qp = qkv + ((size_t)n * HW + qrow) * a.ldq + a.q_off + h * D;
+// Float handles: attention on v_mfma_f32_16x16x4_f32 (float operands, float accumulation). A workgroup of four waves
+// takes QT * 16 queries of one (batch row, head); the waves split the 361 keys (six tiles of 16 each), so that a
+// small batch still fills the chip and a wave's chain is a quarter of the keys. Nothing passes through LDS before the
+// last step: every fragment is read from memory in the order the matrix cores take it.
+// - S^T = K Q^T. A lane's 16-byte load of K is key l16's dims 16c + 4g .. +3 (l16 = lane % 16, g = lane / 16); step j
+//   of the four that contract it takes element j of every lane, dims {16c + 4g + j}, and Q is held in the same order.
+// - A lane then holds keys 4g .. 4g + 3 of one query. Its wave's 96 scores of a query stay in registers, so the
+//   softmax takes one maximum over them and needs no rescaling.
+// - O^T += V^T P^T: step r contracts keys {4g + r}, so P's element r is the operand as it lies. V's rows are read
+//   D / 16 floats per lane at dims (D / 16) l16 .., which makes output row i of tile dt dim (D / 16) i + dt.
+// The four waves' maxima, sums and outputs meet in LDS. Bound: the chain of one wave (its loads and 192 QT MFMAs of 32
+// cycles) at small batches, the matrix cores' float rate (157 TFLOP/s) at large ones. One thread per query on the
+// vector units, keys staged in LDS, before this: 315 -> 18.6 us at 3 rows of 6 heads of 64 dims, 328 -> 41 us at 10 rows
+// of 8 heads (65 TFLOP/s), 76 TFLOP/s at 24 rows of 6.
+constexpr int ATF_NW = 4, ATF_KT = (HW + 15) / 16, ATF_WT = (ATF_KT + ATF_NW - 1) / ATF_NW;  // key tiles, per wave
+// Up to this many (row, head) pairs a workgroup takes 16 queries, beyond it 32 (half the reads of K and V per query):
+// 10.8 against 13.8 us at 6 heads of 64 dims (1 row of b10c384h6), 18.6 against 19.1 at 18, but 23.4 against 20.6 at 40
+// (5 rows of b10c512h8), 45.3 against 41.2 at 80 and 123 against 114 at 256.
+constexpr int ATF_NARROW_HEADS = 20;
+
+template <int D, int QT>
+__global__ __launch_bounds__(ATF_NW * 64) void attn_f32_kernel(const float* __restrict__ qkv,
+                                                               const float* __restrict__ mask, int nheads_total, int H,
+                                                               int KV, int ldq, int q_off, int k_off, int v_off,
+                                                               float scale, float* __restrict__ out, int ldo) {
+  static_assert(D == 16 || D == 32 || D == 64, "head dim");
+  constexpr int KC = D / 16, VW = D / 16, NQ = QT * 16, NQB = (HW + NQ - 1) / NQ;
+  constexpr int OLD = D + 4;
+  typedef float vrow_t __attribute__((ext_vector_type(VW)));
+  __shared__ __align__(16) float Os[ATF_NW * NQ * OLD];
+  __shared__ float Ms[ATF_NW * NQ], Ls[ATF_NW * NQ];
+
+  // The query blocks of one head run on one XCD (workgroup g on XCD g mod 8) and share its L2 for K and V.
+  const int slot = blockIdx.x >> 3, qb = slot % NQB, nh = (slot / NQB) * 8 + (blockIdx.x & 7);
+  if (nh >= nheads_total) return;
+  const int h = nh % H, n = nh / H, kvh = h / (H / KV);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, g = lane >> 4;
+  const float* base = qkv + (size_t)n * HW * ldq;
+  const float* kp = base + k_off + kvh * D + 4 * g;
+  const float* vp = base + v_off + kvh * D + VW * l16;
+  const float* mrow = mask + (size_t)n * HW;
+  const int key0 = wave * ATF_WT * 16;
+
+  // Rows past the board are clamped to the last point: its values are finite wherever the board's are, a key past
+  // the board gets probability 0, and a query past it is not stored.
+  floatx4 qf[QT][KC];
 #pragma unroll
-    for (int d = 0; d < D; d++) q[d] = (float)qp[d] * a.scale;
+  for (int qt = 0; qt < QT; qt++) {
+    const float* qp = base + (size_t)min(qb * NQ + qt * 16 + l16, HW - 1) * ldq + q_off + h * D + 4 * g;
+#pragma unroll
+    for (int c = 0; c < KC; c++) qf[qt][c] = *(const floatx4*)(qp + 16 * c) * scale;
   }
+  floatx4 kf[2][KC];
+  auto load_k = [&](int t, floatx4 (&k)[KC]) {
+    const float* p = kp + (size_t)min(key0 + 16 * t + l16, HW - 1) * ldq;
 #pragma unroll
-  for (int d = 0; d < D; d++) acc[d] = 0.f;
-  float m_run = -FLT_MAX, l_run = 0.f;
-  __shared__ float ks[32 * D], vs[32 * D], kb[32];
-  for (int j0 = 0; j0 < HW; j0 += 32) {
-    const int cnt = min(32, HW - j0);
-    for (int e = tid; e < 32 * D; e += 64) {
-      const int j = e / D, d = e - j * D;
-      float kv = 0.f, vv = 0.f;
-      if (j < cnt) {
-        const T* row = qkv + ((size_t)n * HW + j0 + j) * a.ldq;
-        kv = (float)row[a.k_off + kvh * D + d];
-        vv = (float)row[a.v_off + kvh * D + d];
-      }
-      ks[e] = kv;
-      vs[e] = vv;
+    for (int c = 0; c < KC; c++) k[c] = *(const floatx4*)(p + 16 * c);
+  };
+  vrow_t vf[2][4];
+  auto load_v = [&](int t, vrow_t (&v)[4]) {
+#pragma unroll
+    for (int r = 0; r < 4; r++) v[r] = *(const vrow_t*)(vp + (size_t)min(key0 + 16 * t + 4 * g + r, HW - 1) * ldq);
+  };
+  float mk[ATF_WT][4];
+#pragma unroll
+  for (int t = 0; t < ATF_WT; t++)
+#pragma unroll
+    for (int r = 0; r < 4; r++) mk[t][r] = mrow[min(key0 + 16 * t + 4 * g + r, HW - 1)];
+
+  floatx4 sc[ATF_WT][QT];
+  load_k(0, kf[0]);
+#pragma unroll
+  for (int t = 0; t < ATF_WT; t++) {
+    if (t + 1 < ATF_WT) load_k(t + 1, kf[(t + 1) & 1]);
+    else load_v(0, vf[0]);
+#pragma unroll
+    for (int qt = 0; qt < QT; qt++) sc[t][qt] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < KC; c++)
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+#pragma unroll
+        for (int qt = 0; qt < QT; qt++)
+          sc[t][qt] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[t & 1][c][j], qf[qt][c][j], sc[t][qt], 0, 0, 0);
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const bool on = key0 + 16 * t + 4 * g + r < HW;
+#pragma unroll
+      for (int qt = 0; qt < QT; qt++) sc[t][qt][r] = on ? sc[t][qt][r] + (mk[t][r] * 3e4f - 3e4f) : -1e30f;
     }
-    if (tid < 32) kb[tid] = tid < cnt ? a.mask[(size_t)n * HW + j0 + tid] * 3e4f - 3e4f : 0.f;
-    __syncthreads();
-    float sc[32];
-    float m_blk = m_run;
-#pragma unroll
-    for (int j = 0; j < 32; j++) {
-      if (j < cnt) {
-        float s = 0.f;
-#pragma unroll
-        for (int d = 0; d < D; d++) s += q[d] * ks[j * D + d];
-        s += kb[j];
-        sc[j] = s;
-        m_blk = fmaxf(m_blk, s);
-      }
-    }
-    const float alpha = __expf(m_run - m_blk);
-    l_run *= alpha;
-#pragma unroll
-    for (int d = 0; d < D; d++) acc[d] *= alpha;
-#pragma unroll
-    for (int j = 0; j < 32; j++) {
-      if (j < cnt) {
-        const float p = __expf(sc[j] - m_blk);
-        l_run += p;
-#pragma unroll
-        for (int d = 0; d < D; d++) acc[d] += p * vs[j * D + d];
-      }
-    }
-    m_run = m_blk;
-    __syncthreads();
   }
-  if (in_range) {
-    const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
-    T* o = (T*)a.out + ((size_t)n * HW + qi) * a.ldo + h * D;
+  // The wave's softmax numerators relative to its own maximum, and their sum (both over the four lane groups).
+  float l[QT];
 #pragma unroll
-    for (int d = 0; d < D; d++) o[d] = to_t<T>(acc[d] * inv);
+  for (int qt = 0; qt < QT; qt++) {
+    float m = sc[0][qt][0];
+#pragma unroll
+    for (int t = 0; t < ATF_WT; t++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) m = fmaxf(m, sc[t][qt][r]);
+    m = fmaxf(m, __shfl_xor(m, 16));
+    m = fmaxf(m, __shfl_xor(m, 32));
+    float s = 0.f;
+#pragma unroll
+    for (int t = 0; t < ATF_WT; t++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const float p = __expf(sc[t][qt][r] - m);
+        sc[t][qt][r] = p;
+        s += p;
+      }
+    s += __shfl_xor(s, 16);
+    s += __shfl_xor(s, 32);
+    l[qt] = s;
+    if (g == 0) {
+      Ms[wave * NQ + qt * 16 + l16] = m;
+      Ls[wave * NQ + qt * 16 + l16] = l[qt];
+    }
+  }
+  floatx4 o[VW][QT];
+#pragma unroll
+  for (int dt = 0; dt < VW; dt++)
+#pragma unroll
+    for (int qt = 0; qt < QT; qt++) o[dt][qt] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int t = 0; t < ATF_WT; t++) {
+    if (t + 1 < ATF_WT) load_v(t + 1, vf[(t + 1) & 1]);
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+#pragma unroll
+      for (int dt = 0; dt < VW; dt++)
+#pragma unroll
+        for (int qt = 0; qt < QT; qt++)
+          o[dt][qt] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[t & 1][r][dt], sc[t][qt][r], o[dt][qt], 0, 0, 0);
+  }
+  // Element (dt, r) of a lane is dim VW (4g + r) + dt of its query: 4 VW consecutive dims.
+#pragma unroll
+  for (int qt = 0; qt < QT; qt++) {
+    float* dst = Os + (wave * NQ + qt * 16 + l16) * OLD + 4 * VW * g;
+#pragma unroll
+    for (int e = 0; e < VW; e++) {
+      floatx4 w;
+#pragma unroll
+      for (int k = 0; k < 4; k++) w[k] = o[(4 * e + k) % VW][qt][(4 * e + k) / VW];
+      *(floatx4*)(dst + 4 * e) = w;
+    }
+  }
+  __syncthreads();
+  for (int e = tid; e < NQ * (D / 4); e += ATF_NW * 64) {
+    const int q = e / (D / 4), d = (e % (D / 4)) * 4, qi = qb * NQ + q;
+    float m = Ms[q];
+#pragma unroll
+    for (int w = 1; w < ATF_NW; w++) m = fmaxf(m, Ms[w * NQ + q]);
+    float sum = 0.f;
+    floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < ATF_NW; w++) {
+      const float f = __expf(Ms[w * NQ + q] - m);
+      sum += f * Ls[w * NQ + q];
+      acc += f * *(const floatx4*)(Os + (w * NQ + q) * OLD + d);
+    }
+    if (qi < HW) *(floatx4*)(out + ((size_t)n * HW + qi) * ldo + h * D + d) = acc * (sum > 0.f ? 1.f / sum : 0.f);
   }
 }
 
@@ -1459,19 +1555,26 @@ static void attn_mfma_d(const AttnArgs& a, int B, hipStream_t s) {
            a.v_off, a);
 }
 
-template <typename T, int D>
-static void attn_d(const AttnArgs& a, int B, hipStream_t s) {
-  dim3 grid((HW + 63) / 64, a.H, B);
-  launch_k(attn_kernel<T, D>, grid, 64, 0, s, a);
+template <int D>
+static void attn_f32_d(const AttnArgs& a, int B, hipStream_t s) {
+  const int nh = B * a.H, slots = (nh + 7) / 8 * 8;
+  auto go = [&](auto kernel, int nq) {
+    launch_k(kernel, dim3(slots * ((HW + nq - 1) / nq)), ATF_NW * 64, 0, s, (const float*)a.qkv, a.mask, nh, a.H, a.KV,
+             a.ldq, a.q_off, a.k_off, a.v_off, a.scale, (float*)a.out, a.ldo);
+  };
+  // A query's result does not depend on the queries beside it, so both widths give the same bits.
+  if (nh <= ATF_NARROW_HEADS) go(attn_f32_kernel<D, 1>, 16);
+  else go(attn_f32_kernel<D, 2>, 32);
 }
 
-template <typename T>
-static void attn_t(const AttnArgs& a, int B, hipStream_t s) {
+static void attn_f32(const AttnArgs& a, int B, hipStream_t s) {
   if (a.dq != a.dv) throw std::runtime_error("attention: dq != dv unsupported");
+  if (a.ldq % 4 || a.q_off % 4 || a.k_off % 4 || a.v_off % 4 || a.ldo % 4)  // 16-byte rows
+    throw std::runtime_error("attention: q/k/v and output offsets must be multiples of 4 elements");
   switch (a.dq) {
-    case 16: attn_d<T, 16>(a, B, s); break;
-    case 32: attn_d<T, 32>(a, B, s); break;
-    case 64: attn_d<T, 64>(a, B, s); break;
+    case 16: attn_f32_d<16>(a, B, s); break;
+    case 32: attn_f32_d<32>(a, B, s); break;
+    case 64: attn_f32_d<64>(a, B, s); break;
     default: throw std::runtime_error("attention: head dim must be 16, 32 or 64");
   }
 }
@@ -1493,7 +1596,7 @@ static void attn_mfma_t(const AttnArgs& a, int B, hipStream_t s) {
 void launch_attention(int prec, const AttnArgs& a, int B, hipStream_t s) {
   if (prec == PREC_F16) attn_mfma_t<f16>(a, B, s);
   else if (prec == PREC_BF16) attn_mfma_t<bf16>(a, B, s);
-  else attn_t<float>(a, B, s);
+  else attn_f32(a, B, s);
   KGX_CHECK_LAUNCH();
 }
 
