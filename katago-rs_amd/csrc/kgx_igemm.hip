@@ -847,6 +847,13 @@ void launch_conv_igemm(int prec, int ks, const void* x, int ldx, int IC, const v
       throw std::runtime_error("conv_igemm: unsupported pooling partials");
   }
   const int M = B * HW, kind = igemm_kind(ks, IC, OC, split);
+  if (kind == IG3_48) {
+    if (const int mb = conv_small_mb(ks, IC, icp, OC, M)) {
+      launch_conv_small(prec, mb, x, ldx, w, icp, OC, o, M, Ig3::BN, s);
+      KGX_CHECK_LAUNCH();
+      return;
+    }
+  }
   if (prec == PREC_F16) igemm_dispatch<f16>(kind, x, x_lo, ldx, IC, w, icp, OC, o, M, s);
   else igemm_dispatch<bf16>(kind, x, x_lo, ldx, IC, w, icp, OC, o, M, s);
   KGX_CHECK_LAUNCH();

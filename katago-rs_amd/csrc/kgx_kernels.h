@@ -182,6 +182,12 @@ void conv_igemm_pack_weights(int ks, const float* w, int oc, int ic, std::vector
                              int prec = PREC_F16);
 void launch_conv_igemm(int prec, int ks, const void* x, int ldx, int IC, const void* w, int icp, int OC,
                        const ConvOut& o, int B, hipStream_t s, const void* x_lo = nullptr);
+// The 3x3 convolution of few pixels (kgx_igemm_small.hip): same operands, packed weights (column tiles of pbn) and
+// results as launch_conv_igemm's 48-column 3x3, on tiles of 64 mb pixels x 16 channels; conv_small_mb is 0 where that
+// one runs.
+int conv_small_mb(int ks, int ic, int icp, int oc, int M);
+void launch_conv_small(int prec, int mb, const void* x, int ldx, const void* w, int icp, int OC, const ConvOut& o, int M,
+                       int pbn, hipStream_t s);
 // The value a float becomes as a compute-type operand (round to nearest even), as a float.
 float conv_round_operand(float v, int prec);
 
