@@ -31,7 +31,10 @@ namespace kgx {
 namespace {
 
 constexpr int JCI = kJunctionInner, JCO = kJunctionOuter;
-constexpr int JR = 48;                         // pixels per workgroup (three 16-row MFMA blocks)
+// Pixels per workgroup: IB 16-row MFMA blocks, three where the batch fills the chip with them, one or two below
+// (junction_blocks).
+constexpr int junction_rows(int ib) { return 16 * ib; }
+constexpr int JR48 = junction_rows(3);
 constexpr int JNT = 512;                       // threads: eight waves, two per SIMD
 constexpr int K1 = JCI / 32, K2 = JCO / 32;    // 16x16x32 steps of the exit and the entry product
 constexpr int CB1 = JCO / 16;                  // 16-column blocks of the exit's output
@@ -45,17 +48,18 @@ __host__ __device__ constexpr int junction_welems(int no) { return W2OFF + (no /
 // 192 channels), the exit's float tile [48][384 + 4] and the entry's two float tiles [2][48][NO + 4] (at most
 // the exit's).
 constexpr int LD1 = JCO + 4;
-constexpr int ACTB = (JCO / 64) * 2 * JR * 128;
-constexpr int A1B = (JCI / 64) * 2 * JR * 128, C1B = JR * LD1 * 4, C2B = 2 * JR * (JCI + 4) * 4;
-constexpr int R1B = A1B > C1B ? (A1B > C2B ? A1B : C2B) : (C1B > C2B ? C1B : C2B);
-constexpr int LDSB = ACTB + R1B;
+constexpr int junction_act_bytes(int jr) { return (JCO / 64) * 2 * jr * 128; }
+constexpr int junction_r1_bytes(int jr, bool stem) {
+  const int a1 = (JCI / 64) * 2 * jr * 128, c1 = jr * LD1 * 4, c2 = 2 * jr * (JCI + 4) * 4;
+  const int st = stem ? (jr + 41) * 80 : 0;  // the stem's staged pixel rows and zero row (SRB)
+  const int a = a1 > c1 ? a1 : c1, b = c2 > st ? c2 : st;
+  return a > b ? a : b;
+}
 // Epilogue mappings, the same for every thread (no branch around a memory access, so the compiler's count of the
 // loads in flight stays exact and a later wait for a prefetched weight fragment leaves the trunk's stores in
 // flight): thread t takes channel quads t % G + G q, q < 3, of pixels t / G + R e, for the exit's G = 32 and R = 16
-// (three pixels each) and the entry's G = NO / 12 and R = 512 / G (pixels past 48 skipped at the end). Consecutive
+// (IB pixels each) and the entry's G = NO / 12 and R = 512 / G (pixels past the tile skipped at the end). Consecutive
 // lanes take consecutive quads, so each access of a wave covers whole cache lines.
-constexpr int E1 = 3;
-constexpr int NS = 2;  // weight steps in flight per product (of six per wave)
 static_assert(JNT / 64 == 8 && CB1 == 3 * 8 && K2 == 12, "wave layout assumes 384 and 192 channels");
 
 // The XCD-aware tile order: workgroup g runs on XCD g % 8, and the four 48-pixel tiles of one 192-pixel region go
@@ -81,27 +85,33 @@ __device__ __forceinline__ void lds_barrier() {
 // The stem's packed fragments: [column block][tap] single-plane fragments, then the entry's.
 constexpr int KS3 = 9;                       // the stem's steps: one per tap, 32 channels each
 constexpr int W2STEM = CB1 * KS3 * FRAG;
-constexpr int SR = JR + 40, SRB = 80;        // the stem's staged pixel rows (tile and halos), bytes per LDS row
+constexpr int SRB = 80;                      // bytes per staged pixel row of the stem in LDS
 
 // ACT1: the exit's emission activation (ACT_MISH), or -1: the one eo names, chosen per value at run time. NO: the
 // entry's outputs (192 or 96). A trunk that ends here (eo.y_dead) is read and not stored. STEM: the exit is the
 // network's stem (X: packed input rows of ldx <= 32 channels; eo adds the row's global bias, eo.colbias, instead of
 // a residual). SC2 >= 0: the entry's store case (store_flags of no: SF_Y | SF_EMIT emitting mish, or SF_Y), fixed by
-// the launch so that the kernel holds only that store path; -1: chosen from the arguments.
-template <typename T, int ACT1, int NO, bool STEM, int SC2 = -1>
+// the launch so that the kernel holds only that store path; -1: chosen from the arguments. IB < 3: fewer pixels, whose
+// registers hold more of the weights in flight, with the tiles dealt over all XCDs in order (a board of 48-pixel
+// tiles lies on two).
+template <typename T, int ACT1, int NO, bool STEM, int IB, int SC2 = -1>
 __global__ __launch_bounds__(JNT, 1) void junction_kernel(const T* __restrict__ X, const T* __restrict__ Xlo, int ldx,
                                                           const T* __restrict__ W, int M, ConvOut eo, ConvOut no) {
   typedef typename std::conditional<std::is_same<T, f16>::value, half8, bf16x8>::type frag_t;
   static_assert(NO == 192 || NO == 96, "entry outputs");
+  constexpr int JR = junction_rows(IB), ACTB = junction_act_bytes(JR), E1 = IB;
+  // Weight steps in flight per product (of six per wave, the stem's nine).
+  constexpr int NS = IB == 3 ? 2 : IB == 2 ? 3 : 4;
+  constexpr int SR = JR + 40;                // the stem's staged pixel rows (tile and halos)
   constexpr int W2 = STEM ? W2STEM : W2OFF;  // the entry's fragments
   constexpr int CB2 = NO / 16, LD2 = NO + 4;
   constexpr int G2 = NO / 12, R2 = JNT / G2, E2 = (JR + R2 - 1) / R2;  // the entry epilogue's mapping
-  __shared__ __align__(1024) char smem[LDSB];
+  __shared__ __align__(1024) char smem[ACTB + junction_r1_bytes(JR, STEM)];
   char* const act = smem;
   char* const r1 = smem + ACTB;
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r16 = lane & 15, g4 = lane >> 4;
-  const int m0 = junction_tile(blockIdx.x) * JR;
+  const int m0 = (IB == 3 ? junction_tile(blockIdx.x) : (int)blockIdx.x) * JR;
   if (m0 >= M) {  // an idle workgroup still touches its share of the next launch's weights
     l2_touch_keep(l2_touch(no.pf, no.pf_bytes, tid));
     return;
@@ -147,9 +157,9 @@ __global__ __launch_bounds__(JNT, 1) void junction_kernel(const T* __restrict__ 
     }
   };
 
-  floatx4 acc[3][3];
+  floatx4 acc[IB][3];
 #pragma unroll
-  for (int i = 0; i < 3; i++)
+  for (int i = 0; i < IB; i++)
 #pragma unroll
     for (int j = 0; j < 3; j++) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
   if constexpr (STEM) {
@@ -171,9 +181,9 @@ __global__ __launch_bounds__(JNT, 1) void junction_kernel(const T* __restrict__ 
     else if (tid < SR * 4 + SRB / 16) *(u32x4*)(r1 + SR * SRB + (tid - SR * 4) * 16) = u32x4{0, 0, 0, 0};  // zero row
     // Tap validity of this lane's pixels (bit t: the neighbour at tap t is on the board); off-board neighbours,
     // and pixels past M, read the zero row.
-    unsigned vmask[3];
+    unsigned vmask[IB];
 #pragma unroll
-    for (int i = 0; i < 3; i++) {
+    for (int i = 0; i < IB; i++) {
       const int m = m0 + 16 * i + r16;
       unsigned bits = 0;
       if (m < M) {
@@ -185,11 +195,11 @@ __global__ __launch_bounds__(JNT, 1) void junction_kernel(const T* __restrict__ 
       vmask[i] = bits;
     }
     lds_barrier();
-    frag_t a[2][3];
+    frag_t a[2][IB];
     auto load_a = [&](int set, int t) {
       const int shift = (t / 3 - 1) * POS + (t % 3 - 1);
 #pragma unroll
-      for (int i = 0; i < 3; i++) {
+      for (int i = 0; i < IB; i++) {
         const int row = (vmask[i] >> t) & 1 ? 16 * i + r16 + 20 + shift : SR;
         a[set][i] = *(const frag_t*)(r1 + row * SRB + g4 * 16);
       }
@@ -200,7 +210,7 @@ __global__ __launch_bounds__(JNT, 1) void junction_kernel(const T* __restrict__ 
       if (t + 1 < KS3) load_a((t + 1) & 1, t + 1);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int i = 0; i < 3; i++)
+      for (int i = 0; i < IB; i++)
 #pragma unroll
         for (int j = 0; j < 3; j++) acc[i][j] = mfma(a[t & 1][i], b1[t % NS][j], acc[i][j]);
       __builtin_amdgcn_sched_barrier(0);
@@ -220,7 +230,7 @@ __global__ __launch_bounds__(JNT, 1) void junction_kernel(const T* __restrict__ 
     };
 #pragma unroll
     for (int k = 0; k < NS; k++) load_b1(k, k);
-    // The exit's operand straight into LDS: 36 loads of 8 pixel rows x 128 bytes (64-channel slice kp, plane pl,
+    // The exit's operand straight into LDS: 12 IB loads of 8 pixel rows x 128 bytes (64-channel slice kp, plane pl,
     // rows 8 grp ..), lane i filling row 8 grp + i / 8 at stored chunk i % 8 from source chunk (i % 8) ^ swizzle.
     // Rows past M lie beyond the buffer range and read as zero.
     {
@@ -228,10 +238,10 @@ __global__ __launch_bounds__(JNT, 1) void junction_kernel(const T* __restrict__ 
       const T* xb = X + (size_t)m0 * ldx;
       const T* xlb = Xlo + (size_t)m0 * ldx;
 #pragma unroll
-      for (int u = 0; u < 5; u++) {
+      for (int u = 0; u < (12 * IB + 7) / 8; u++) {
         const int q = u * 8 + wv;
-        if (q < 36) {
-          const int kp = q / 12, pl = (q / 6) & 1, grp = q % 6;
+        if (q < 12 * IB) {
+          const int kp = q / (4 * IB), pl = (q / (2 * IB)) & 1, grp = q % (2 * IB);
           const int row = grp * 8 + (lane >> 3), sc = (lane & 7) ^ ((row >> 1) & 7);
           lds_load16(pl ? xlb : xb, nbytes, r1 + ((kp * 2 + pl) * JR + grp * 8) * 128, row * rb + kp * 128 + sc * 16);
         }
@@ -242,10 +252,10 @@ __global__ __launch_bounds__(JNT, 1) void junction_kernel(const T* __restrict__ 
     __syncthreads();
 
     {
-      frag_t ah[2][3], al[2][3];
+      frag_t ah[2][IB], al[2][IB];
       auto load_a1 = [&](int set, int ks) {
 #pragma unroll
-        for (int i = 0; i < 3; i++) {
+        for (int i = 0; i < IB; i++) {
           ah[set][i] = afrag(r1, i, ks, 0);
           al[set][i] = afrag(r1, i, ks, 1);
         }
@@ -257,15 +267,15 @@ __global__ __launch_bounds__(JNT, 1) void junction_kernel(const T* __restrict__ 
         if (ks + 1 < K1) load_a1(s ^ 1, ks + 1);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int i = 0; i < 3; i++)
+        for (int i = 0; i < IB; i++)
 #pragma unroll
           for (int j = 0; j < 3; j++) acc[i][j] = mfma(al[s][i], b1[ks % NS][j][0], acc[i][j]);
 #pragma unroll
-        for (int i = 0; i < 3; i++)
+        for (int i = 0; i < IB; i++)
 #pragma unroll
           for (int j = 0; j < 3; j++) acc[i][j] = mfma(ah[s][i], b1[ks % NS][j][1], acc[i][j]);
 #pragma unroll
-        for (int i = 0; i < 3; i++)
+        for (int i = 0; i < IB; i++)
 #pragma unroll
           for (int j = 0; j < 3; j++) acc[i][j] = mfma(ah[s][i], b1[ks % NS][j][0], acc[i][j]);
         __builtin_amdgcn_sched_barrier(0);
@@ -295,7 +305,7 @@ __global__ __launch_bounds__(JNT, 1) void junction_kernel(const T* __restrict__ 
   lds_barrier();
   float* const C1 = (float*)r1;
 #pragma unroll
-  for (int i = 0; i < 3; i++)
+  for (int i = 0; i < IB; i++)
 #pragma unroll
     for (int j = 0; j < 3; j++)
 #pragma unroll
@@ -356,15 +366,15 @@ __global__ __launch_bounds__(JNT, 1) void junction_kernel(const T* __restrict__ 
     *(uint2*)(d + JR * 128) = *(const uint2*)lo;
   };
 
-  floatx4 acc2[3][3];
+  floatx4 acc2[IB][3];
 #pragma unroll
-  for (int i = 0; i < 3; i++)
+  for (int i = 0; i < IB; i++)
 #pragma unroll
     for (int j = 0; j < 3; j++) acc2[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-  frag_t ah[2][3], al[2][3];
+  frag_t ah[2][IB], al[2][IB];
   auto load_a2 = [&](int set, int p) {
 #pragma unroll
-    for (int i = 0; i < 3; i++) {
+    for (int i = 0; i < IB; i++) {
       ah[set][i] = afrag(act, i, kstep(p), 0);
       al[set][i] = afrag(act, i, kstep(p), 1);
     }
@@ -372,15 +382,15 @@ __global__ __launch_bounds__(JNT, 1) void junction_kernel(const T* __restrict__ 
   auto mma2 = [&](int p) {
     const int s = p & 1;
 #pragma unroll
-    for (int i = 0; i < 3; i++)
+    for (int i = 0; i < IB; i++)
 #pragma unroll
       for (int j = 0; j < 3; j++) acc2[i][j] = mfma(al[s][i], b2[p % NS][j][0], acc2[i][j]);
 #pragma unroll
-    for (int i = 0; i < 3; i++)
+    for (int i = 0; i < IB; i++)
 #pragma unroll
       for (int j = 0; j < 3; j++) acc2[i][j] = mfma(ah[s][i], b2[p % NS][j][1], acc2[i][j]);
 #pragma unroll
-    for (int i = 0; i < 3; i++)
+    for (int i = 0; i < IB; i++)
 #pragma unroll
       for (int j = 0; j < 3; j++) acc2[i][j] = mfma(ah[s][i], b2[p % NS][j][0], acc2[i][j]);
   };
@@ -405,14 +415,16 @@ __global__ __launch_bounds__(JNT, 1) void junction_kernel(const T* __restrict__ 
       load_a2(1, 2 * b + 1);
       if (b < 2) {
         epi1(act_c, b + 1, 0);
-        epi1(act_c, b + 1, 1);
+        if constexpr (IB > 2) epi1(act_c, b + 1, 1);
       }
       __builtin_amdgcn_sched_barrier(0);
-      if (2 * b + NS < K2 / 2) load_b2(0, 2 * b + NS);
+      if (2 * b + NS < K2 / 2) load_b2((2 * b) % NS, 2 * b + NS);
       mma2(2 * b + 1);
-      if (b < 2) epi1(act_c, b + 1, 2);
+      if constexpr (IB > 1) {
+        if (b < 2) epi1(act_c, b + 1, IB - 1);
+      }
       __builtin_amdgcn_sched_barrier(0);
-      if (2 * b + 1 + NS < K2 / 2) load_b2(1, 2 * b + 1 + NS);
+      if (2 * b + 1 + NS < K2 / 2) load_b2((2 * b + 1) % NS, 2 * b + 1 + NS);
       if (b < 2) lds_barrier();
     }
   };
@@ -422,7 +434,7 @@ __global__ __launch_bounds__(JNT, 1) void junction_kernel(const T* __restrict__ 
   float* const C2 = (float*)r1;
   if (c2own) {
 #pragma unroll
-    for (int i = 0; i < 3; i++)
+    for (int i = 0; i < IB; i++)
 #pragma unroll
       for (int j = 0; j < 3; j++)
 #pragma unroll
@@ -462,8 +474,11 @@ __global__ __launch_bounds__(JNT, 1) void junction_kernel(const T* __restrict__ 
 
 int junction_tile_of(int g) { return junction_tile(g); }
 
+// 16-row blocks per workgroup over M pixels: the fewest whose workgroups all run at once (one per CU).
+int junction_blocks(int M) { return M <= 256 * junction_rows(1) ? 1 : M <= 256 * junction_rows(2) ? 2 : 3; }
+
 int junction_grid(int M) {
-  const int regions = (M + 4 * JR - 1) / (4 * JR);
+  const int regions = (M + 4 * JR48 - 1) / (4 * JR48);
   return 32 * ((regions + 7) / 8);
 }
 
@@ -531,13 +546,21 @@ void launch_junction(int prec, const void* x, const void* x_lo, int ldx, const v
   const int sc2 = !mish ? -1
                   : entry_oc == kJunctionInner && fl2 == (SF_Y | SF_EMIT) && no.emit.act == ACT_MISH ? SF_Y | SF_EMIT
                   : entry_oc == kJunctionHead && fl2 == SF_Y ? SF_Y : -1;
-  auto go = [&](auto tc, auto noc) {
+  const int ib = junction_blocks(M);
+  auto go_ib = [&](auto tc, auto noc, auto ibc) {
     typedef decltype(tc) TT;
-    constexpr int N = decltype(noc)::value;
+    constexpr int N = decltype(noc)::value, IB = decltype(ibc)::value;
     constexpr int SPEC2 = N == kJunctionInner ? SF_Y | SF_EMIT : SF_Y;
-    launch_k(!mish ? junction_kernel<TT, -1, N, false>
-                   : sc2 >= 0 ? junction_kernel<TT, ACT_MISH, N, false, SPEC2> : junction_kernel<TT, ACT_MISH, N, false>,
-             junction_grid(M), JNT, 0, s, (const TT*)x, (const TT*)x_lo, ldx, (const TT*)w, M, eo, no);
+    launch_k(!mish ? junction_kernel<TT, -1, N, false, IB>
+                   : sc2 >= 0 ? junction_kernel<TT, ACT_MISH, N, false, IB, SPEC2>
+                              : junction_kernel<TT, ACT_MISH, N, false, IB>,
+             IB == 3 ? junction_grid(M) : (M + junction_rows(IB) - 1) / junction_rows(IB), JNT, 0, s, (const TT*)x,
+             (const TT*)x_lo, ldx, (const TT*)w, M, eo, no);
+  };
+  auto go = [&](auto tc, auto noc) {
+    if (ib == 1) go_ib(tc, noc, std::integral_constant<int, 1>());
+    else if (ib == 2) go_ib(tc, noc, std::integral_constant<int, 2>());
+    else go_ib(tc, noc, std::integral_constant<int, 3>());
   };
   typedef std::integral_constant<int, kJunctionInner> Inner;
   typedef std::integral_constant<int, kJunctionHead> Head;
@@ -570,12 +593,20 @@ void launch_stem_junction(int prec, const void* x, int ldx, const void* w, const
   const int M = B * HW;
   const bool mish = eo.emit.act == ACT_MISH;
   const bool spec2 = mish && store_flags(no) == (SF_Y | SF_EMIT) && no.emit.act == ACT_MISH;
-  auto go = [&](auto tc) {
+  const int ib = junction_blocks(M);
+  auto go_ib = [&](auto tc, auto ibc) {
     typedef decltype(tc) TT;
-    launch_k(!mish ? junction_kernel<TT, -1, kJunctionInner, true>
-                   : spec2 ? junction_kernel<TT, ACT_MISH, kJunctionInner, true, SF_Y | SF_EMIT>
-                           : junction_kernel<TT, ACT_MISH, kJunctionInner, true>,
-             junction_grid(M), JNT, 0, s, (const TT*)x, (const TT*)x, ldx, (const TT*)w, M, eo, no);
+    constexpr int IB = decltype(ibc)::value;
+    launch_k(!mish ? junction_kernel<TT, -1, kJunctionInner, true, IB>
+                   : spec2 ? junction_kernel<TT, ACT_MISH, kJunctionInner, true, IB, SF_Y | SF_EMIT>
+                           : junction_kernel<TT, ACT_MISH, kJunctionInner, true, IB>,
+             IB == 3 ? junction_grid(M) : (M + junction_rows(IB) - 1) / junction_rows(IB), JNT, 0, s, (const TT*)x,
+             (const TT*)x, ldx, (const TT*)w, M, eo, no);
+  };
+  auto go = [&](auto tc) {
+    if (ib == 1) go_ib(tc, std::integral_constant<int, 1>());
+    else if (ib == 2) go_ib(tc, std::integral_constant<int, 2>());
+    else go_ib(tc, std::integral_constant<int, 3>());
   };
   if (prec == PREC_F16) go(f16());
   else go(bf16());

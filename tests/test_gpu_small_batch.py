@@ -31,3 +31,19 @@ def test_rows_equal_the_large_tiles(kgx, synth, oracle, prec, trunk, mid, act, b
     r = [0, n - 1]
     check(full[r], oracle.Model(mb).forward(sp[r], gl[r]), net.P, net.S, prec, "small launches",
           emulated(oracle, mb, prec, sp[r], gl[r]))
+
+
+@pytest.mark.parametrize("prec", ["f16", "bf16"])
+@pytest.mark.parametrize("act", ["ACTIVATION_MISH", "ACTIVATION_RELU"])
+def test_junction_rows_equal_the_48_pixel_tiles(kgx, synth, prec, act):
+    """Junctions, the stem and the head junction on 16-pixel (up to 11 rows), 32-pixel (up to 22) and 48-pixel tiles."""
+    print(f"small junctions: {prec}, {act}", flush=True)
+    arch = synth.Arch("t-smalljunction", 14, 384, [("nbt", 192, [("res", 192)]), ("nbt", 192, [("gpool", 192, 64)])] * 2,
+                      mid_c=192, gpool_c=64, act=act)
+    n = 23
+    sp, gl, _ = synth.make_inputs(n, 13, board_sizes=[19, 13, 9])
+    h = kgx.Handle(kgx.Net(synth.write_model(arch, 8)), n, prec)
+    full = h.forward(sp, gl)
+    for k in (1, 2, 11, 12, 22):
+        assert np.array_equal(h.forward(sp[:k], gl[:k]), full[:k]), k
+    h.close()
