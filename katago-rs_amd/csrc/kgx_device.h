@@ -228,6 +228,18 @@ __device__ __forceinline__ int l2_touch(const char* p, int nbytes, int tid) {
 }
 __device__ __forceinline__ void l2_touch_keep(int v) { asm volatile("" ::"v"(v)); }
 
+// Waits for this wave's LDS accesses, then for every wave: nothing else. A fence (__syncthreads()) would also wait
+// for the wave's loads and stores in flight (the weight prefetch, the trunk's stores). The compiler moves no memory
+// access across the clobbers, nor the clobbers across the barrier.
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("" ::: "memory");
+}
+
 // Winograd F(TM x TM, 3x3) geometry on the 19x19 board.
 template <int TM>
 struct Wino {

@@ -70,18 +70,6 @@ __host__ __device__ inline int junction_tile(int g) {
   return 4 * (xcd + 8 * (slot >> 2)) + (slot & 3);
 }
 
-// Waits for this wave's LDS accesses, then for every wave: nothing else. A fence (__syncthreads()) would also wait
-// for the wave's loads and stores in flight (the weight prefetch, the trunk's stores). The compiler moves no memory
-// access across the clobbers, nor the clobbers across the barrier.
-__device__ __forceinline__ void lds_barrier() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
-  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_sched_barrier(0);
-  asm volatile("" ::: "memory");
-}
-
 // The stem's packed fragments: [column block][tap] single-plane fragments, then the entry's.
 constexpr int KS3 = 9;                       // the stem's steps: one per tap, 32 channels each
 constexpr int W2STEM = CB1 * KS3 * FRAG;

@@ -188,6 +188,10 @@ void launch_conv_igemm(int prec, int ks, const void* x, int ldx, int IC, const v
 int conv_small_mb(int ks, int ic, int icp, int oc, int M);
 void launch_conv_small(int prec, int mb, const void* x, int ldx, const void* w, int icp, int OC, const ConvOut& o, int M,
                        int pbn, hipStream_t s);
+// Float 3x3 convolution on bf16 matrix cores (kgx_split.hip): x float NHWC rows of ldx (IC % 8 == 0), w the upload of
+// conv_split_pack_weights, OC % 4 == 0.
+void conv_split_pack_weights(const float* w, int oc, int ic, std::vector<float>& out);
+void launch_conv_split(const float* x, int ldx, int IC, const void* w, int OC, const ConvOut& o, int B, hipStream_t s);
 // The value a float becomes as a compute-type operand (round to nearest even), as a float.
 float conv_round_operand(float v, int prec);
 

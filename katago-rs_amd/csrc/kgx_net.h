@@ -160,7 +160,7 @@ class Net {
 
   int t_pad(int B) const;  // Winograd tiles of B rows, padded to the GEMM's row tile
 
-  enum ConvMode { CONV_IGEMM, CONV_WINO2, CONV_WINO4 };
+  enum ConvMode { CONV_IGEMM, CONV_SPLIT, CONV_WINO2, CONV_WINO4 };
   int device_, max_batch_, prec_;
   const Net* primary_ = nullptr;
   std::vector<std::pair<const void*, size_t>> uploads_;  // device copies of the weights, in upload order

@@ -37,18 +37,19 @@ uint16_t f32_to_bf16_bits(float f) {  // round to nearest even
 
 Net::Net(const ModelDesc& m, int device, int max_batch, int prec) : device_(device), max_batch_(max_batch), prec_(prec) {
   KGX_HIP(hipSetDevice(device));
-  // Convolution algorithm. Float operands: Winograd F(4x4,3x3), the reference's. 16-bit operands: implicit GEMM
-  // for 1x1 and 3x3 (no transform traffic; only activations and weights are rounded). KGX_CONV=igemm|wino2|wino4
-  // overrides (igemm needs 16-bit operands; wino2 is F(2x2,3x3), whose transformed values stay small enough for
+  // Convolution algorithm. Float operands: the direct sum of three-plane bf16 splits (kgx_split.hip) where the shape
+  // fits it, else Winograd F(4x4,3x3), the reference's. 16-bit operands: implicit GEMM for 1x1 and 3x3 (no transform
+  // traffic; only activations and weights are rounded). KGX_CONV=igemm|wino2|wino4 overrides (igemm needs 16-bit
+  // operands; wino4 is F(4x4,3x3) for every shape; wino2 is F(2x2,3x3), whose transformed values stay small enough for
   // 16-bit operands).
-  conv_mode_ = prec == PREC_F32 ? CONV_WINO4 : CONV_IGEMM;
+  conv_mode_ = prec == PREC_F32 ? CONV_SPLIT : CONV_IGEMM;
   if (const char* e = std::getenv("KGX_CONV")) {
     const std::string v = e;
     if (v == "wino4") conv_mode_ = CONV_WINO4;
     else if (v == "wino2") conv_mode_ = CONV_WINO2;
     else if (v == "igemm" && prec != PREC_F32) conv_mode_ = CONV_IGEMM;
   }
-  wino_tm_ = conv_mode_ == CONV_WINO4 ? 4 : 2;
+  wino_tm_ = conv_mode_ == CONV_WINO4 || conv_mode_ == CONV_SPLIT ? 4 : 2;
   // Nested-bottleneck junctions in one launch; KGX_JUNCTION=0 plans the two convolutions separately.
   if (const char* e = std::getenv("KGX_JUNCTION")) junctions_ = std::string(e) != "0";
   // Each convolution touches the next one's weights into L2 during its epilogue; KGX_L2_PREFETCH=0 turns it off.
@@ -350,6 +351,23 @@ std::shared_ptr<ConvOut> Net::emit_conv(const ConvDesc& c, const void* x, int ld
     op.w = dW;
     op.w_bytes = w.size() * tsize();
     op.pf_sink = out;
+    ops_.push_back(op);
+    return out;
+  }
+  if (k3 && conv_mode_ == CONV_SPLIT && !nchw && c.ic % 8 == 0 && ldx % 4 == 0 && c.oc % 4 == 0 &&
+      (!o.y || o.ldy % 4 == 0) && (!o.yt || o.ldyt % 4 == 0) && (!o.colbias || o.ld_colbias % 4 == 0) && !o.pool.psum) {
+    std::vector<float> w;
+    conv_split_pack_weights(c.w.data(), c.oc, c.ic, w);
+    const float* dW = upload_f(w);
+    const float* xf = (const float*)x;
+    Op op;
+    op.launch = [=](hipStream_t s, int B) { launch_conv_split(xf, ldx, ic, dW, oc, *out, B, s); };
+    op.cls = "conv3x3_split";
+    op.flops_row = 2.0 * 9 * HW * ic * oc;
+    op.bytes_row = in_bytes + out_bytes;
+    op.bytes_fixed = 9.0 * ic * oc * 6;
+    op.out = out;
+    op.out_c = oc;
     ops_.push_back(op);
     return out;
   }

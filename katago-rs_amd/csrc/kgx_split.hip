@@ -1,0 +1,350 @@
+// Float 3x3 convolutions on the bf16 matrix cores. Every float operand is split into three bf16 planes, x = h + m + l
+// (each the rounding of what the planes before it leave: 24 significant bits, float's exponent range), and a product
+// is taken as l h + m m + m h + h l + h m + h h with float accumulation; the terms left out are below 2^-26 of the
+// product. Six v_mfma_f32_16x16x32_bf16 take 96 cycles where v_mfma_f32_16x16x4_f32 takes 256 for the same products,
+// and the direct sum has neither the transforms' traffic of Winograd F(4x4,3x3) nor its loss of accuracy.
+//
+// A workgroup computes 16 MB pixels x 16 NB channels. Per chunk of 64 input channels it stages the pixel rows (tile and
+// a halo of 20, as kgx_igemm.hip) in LDS as three planes, split in registers on the way, in two buffers with one
+// barrier per chunk; all nine taps read them there. Four pairs of waves split the chunk's 18 (tap, 32-channel) steps:
+// pair w takes steps w, w + 4, w + 8, w + 12 and half of the products of step 16 + w / 2, so a weight fragment is read
+// by one pair, straight from memory into registers (packed in fragment order, one 1 KB load each, one step ahead), and
+// never passes through LDS. The pairs' sums are added through LDS in order, which the tile's size does not change: a
+// row's results do not depend on the batch.
+//
+// 192 -> 192 channels at 16 boards (96 x 48 tiles, 244 workgroups): 23.5 us, against 53 us of input transform, 36 point
+// GEMMs and output transform (F(4x4,3x3)); 128 -> 128 at 8 boards (48 x 32): 9.1 against 37 us. The MFMAs are 12 us of
+// the first; splitting the operands costs 2.5 us of VALU time, the first stage and the epilogue 4.
+// An infinite operand gives NaN where it is read (its second plane is inf - inf).
+#include "kgx_device.h"
+
+#include <cstring>
+#include <vector>
+
+namespace kgx {
+
+namespace {
+
+constexpr int PNT = 512, PCH = 64, PSTEPS = 18, PHALO = POS + 1;
+constexpr int PFRAG = 64 * 8;  // elements of a packed weight fragment
+
+// x as three bf16 planes, eight values at a time (16 bytes per plane).
+__device__ __forceinline__ void split3(const floatx4 (&x)[2], u32x4 (&p)[3]) {
+  typedef float floatx2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    floatx2 v = {x[k >> 1][(k & 1) * 2], x[k >> 1][(k & 1) * 2 + 1]};
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+      const unsigned u = __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf16x2));
+      p[q][k] = u;
+      if (q < 2) {
+        v[0] -= __builtin_bit_cast(float, u << 16);
+        v[1] -= __builtin_bit_cast(float, u & 0xffff0000u);
+      }
+    }
+  }
+}
+
+template <int MB, int NB, int SC>
+__global__ __launch_bounds__(PNT, 1) void conv3_split_kernel(const float* __restrict__ X, int ldx, int IC,
+                                                             const bf16* __restrict__ W, int nch, int OC, int M, int ntl,
+                                                             ConvOut o) {
+  // Two waves per step share: over the rows, or over the columns of the tile that is too wide or too short for that.
+  constexpr int WM = MB == 6 && NB < 4 ? 2 : 1, WN = 2 / WM, WB = MB / WM, WC = NB / WN;
+  constexpr int BM = 16 * MB, BN = 16 * NB, AR = BM + 2 * PHALO;
+  constexpr int PLB = (AR + 1) * 128, BUF = 3 * PLB;  // bytes of a chunk's plane (its last row zero) and of a chunk
+  constexpr int LDC = BN + 4, CB = 4 * BM * LDC * 4;
+  __shared__ __align__(128) char smem[2 * BUF > CB ? 2 * BUF : CB];
+  const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wv = wid & 3, wr = WM == 2 ? (wid >> 2) * WB * 16 : 0, wc = WN == 2 ? (wid >> 2) * WC : 0;  // steps, row, block
+  const int r16 = lane & 15, g4 = lane >> 4;
+  // The column tiles of a pixel tile on one XCD (workgroup g runs on XCD g mod 8): they share its L2 for the rows.
+  const int slot = blockIdx.x >> 3, u = slot / ntl, nt = slot - u * ntl, mt = u * 8 + (blockIdx.x & 7);
+  const int m0 = mt * BM, n0 = nt * BN;
+  if (m0 >= M) return;
+
+  // Staging: 8 channels of one row per task.
+  constexpr int SV = (AR * 8 + PNT - 1) / PNT;
+  floatx4 st[SV][2];
+  auto load = [&](int kc) {
+#pragma unroll
+    for (int v = 0; v < SV; v++) {
+      const int t = tid + PNT * v, row = t >> 3, c = kc * PCH + (t & 7) * 8, gr = m0 - PHALO + row;
+      const bool ok = gr >= 0 && gr < M && c < IC;
+      const float* p = X + (size_t)min(max(gr, 0), M - 1) * ldx + (c < IC ? c : 0);
+      st[v][0] = *(const floatx4*)p;
+      st[v][1] = *(const floatx4*)(p + 4);
+      if (!ok) st[v][0] = st[v][1] = floatx4{0.f, 0.f, 0.f, 0.f};
+    }
+  };
+  auto store = [&](int buf) {
+#pragma unroll
+    for (int v = 0; v < SV; v++) {
+      const int t = tid + PNT * v, row = t >> 3;
+      u32x4 p[3];
+      // (Pinned here: hoisted to the loads, the split would wait for them.)
+      asm volatile("" : "+v"(st[v][0]), "+v"(st[v][1]));
+      split3(st[v], p);
+      if (row < AR) {
+        char* d = smem + buf * BUF + row * 128 + (((t & 7) ^ ((row >> 1) & 7)) * 16);
+#pragma unroll
+        for (int q = 0; q < 3; q++) *(u32x4*)(d + q * PLB) = p[q];
+      }
+    }
+  };
+  load(0);
+
+  // Weight fragments (16-column block, chunk, step, plane); blocks past OC are packed as zeros.
+  bf16x8 b0[WC][3], b1[WC][3];
+  const bf16* const wb = W + (size_t)(nt * NB + wc) * nch * PSTEPS * 3 * PFRAG + lane * 8;
+  auto load_b = [&](bf16x8 (&d)[WC][3], int kc, int s) {
+#pragma unroll
+    for (int j = 0; j < WC; j++)
+#pragma unroll
+      for (int q = 0; q < 3; q++) d[j][q] = *(const bf16x8*)(wb + (((size_t)j * nch + kc) * PSTEPS + s) * 3 * PFRAG + q * PFRAG);
+  };
+  load_b(b0, 0, wv);
+
+  // Tap validity of this lane's pixels (bit t: the neighbour at tap t is on the board); others read the zero row.
+  unsigned vmask[WB];
+#pragma unroll
+  for (int i = 0; i < WB; i++) {
+    const int m = m0 + wr + i * 16 + r16;
+    const int p = m % HW, y = p / POS, x = p - y * POS;
+    unsigned bits = m < M ? 0x1ff : 0;
+    if (y == 0) bits &= ~0x007u;
+    if (y == POS - 1) bits &= ~0x1c0u;
+    if (x == 0) bits &= ~0x049u;
+    if (x == POS - 1) bits &= ~0x124u;
+    vmask[i] = bits;
+  }
+  if (tid < 48) *(u32x4*)(smem + (tid >> 3) * PLB + AR * 128 + (tid & 7) * 16) = u32x4{0, 0, 0, 0};
+
+  floatx4 acc[WB][WC];
+#pragma unroll
+  for (int i = 0; i < WB; i++)
+#pragma unroll
+    for (int j = 0; j < WC; j++) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+
+  // The pixel fragments of step s (tap s / 2, channels 32 (s % 2) .. + 32): their addresses, then a plane at a time.
+  bf16x8 a[WB][3];
+  int aoff[WB];
+  auto set_a = [&](int buf, int s) {
+    const int t = s >> 1, kc = (s & 1) * 4 + g4, dy = t / 3, shift = (dy - 1) * POS + (t - 3 * dy - 1);
+#pragma unroll
+    for (int i = 0; i < WB; i++) {
+      const int row = (vmask[i] >> t) & 1 ? wr + i * 16 + r16 + PHALO + shift : AR;
+      aoff[i] = buf * BUF + row * 128 + ((kc ^ ((row >> 1) & 7)) * 16);
+    }
+  };
+  auto load_a = [&](auto pl) {
+    constexpr int q = decltype(pl)::value;
+#pragma unroll
+    for (int i = 0; i < WB; i++) a[i][q] = *(const bf16x8*)(smem + aoff[i] + q * PLB);
+  };
+  auto prod = [&](const bf16x8 (&d)[WC][3], auto pa, auto pb) {
+#pragma unroll
+    for (int i = 0; i < WB; i++)
+#pragma unroll
+      for (int j = 0; j < WC; j++)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i][decltype(pa)::value], d[j][decltype(pb)::value],
+                                                            acc[i][j], 0, 0, 0);
+  };
+  typedef std::integral_constant<int, 0> H;
+  typedef std::integral_constant<int, 1> Mi;
+  typedef std::integral_constant<int, 2> L;
+
+  // Rolled loops: straight-line code of all steps, each executed once, ran no faster than its instructions arrive in the
+  // cold instruction cache (29 against 26 us). Two weight fragment sets take the steps in turn. A plane of the next
+  // step's pixel fragments is read as soon as this step's products of it are issued.
+  const int half = 16 + (wv >> 1);
+  // One of the three thirds of a step's weight fragments (a plane).
+  auto load_bp = [&](bf16x8 (&d)[WC][3], int kc, int s, auto pl) {
+    constexpr int q = decltype(pl)::value;
+#pragma unroll
+    for (int j = 0; j < WC; j++) d[j][q] = *(const bf16x8*)(wb + (((size_t)j * nch + kc) * PSTEPS + s) * 3 * PFRAG + q * PFRAG);
+  };
+  // The scheduler's pattern of a phase: its LDS and memory reads spread between the MFMAs, which issue meanwhile.
+  auto spread = [&](auto nm, auto nv) {
+#pragma unroll
+    for (int k = 0; k < decltype(nm)::value; k++) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+      if (k < WB) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      if (k < WC) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x002, decltype(nv)::value, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // The step whose fragments are in d (its H plane of the pixels read here), loading step sn into dn and its pixels.
+  auto step = [&](const bf16x8 (&d)[WC][3], bf16x8 (&dn)[WC][3], int kc, int buf, int sn) {
+    __builtin_amdgcn_sched_barrier(0);
+    load_a(H{});
+    set_a(buf, sn);
+    load_bp(dn, kc, sn, L{});
+    prod(d, L{}, H{});
+    spread(std::integral_constant<int, WB * WC / 2>{}, std::integral_constant<int, 8>{});
+    load_a(L{});
+    load_bp(dn, kc, sn, Mi{});
+    prod(d, Mi{}, Mi{});
+    prod(d, Mi{}, H{});
+    spread(std::integral_constant<int, WB * WC>{}, std::integral_constant<int, 1>{});
+    load_a(Mi{});
+    load_bp(dn, kc, sn, H{});
+    prod(d, H{}, L{});
+    prod(d, H{}, Mi{});
+    prod(d, H{}, H{});
+    spread(std::integral_constant<int, WB * WC * 3 / 2>{}, std::integral_constant<int, 1>{});
+  };
+  store(0);
+#pragma unroll 1
+  for (int kc = 0; kc < nch; kc++) {
+    const int buf = kc & 1;
+    const bool more = kc + 1 < nch;
+    lds_barrier();
+    if (more) load(kc + 1);
+    set_a(buf, wv);
+    load_a(L{});
+    load_a(Mi{});
+#pragma unroll 1
+    for (int j = 0; j < 4; j += 2) {
+      step(b0, b1, kc, buf, wv + 4 * j + 4);
+      step(b1, b0, kc, buf, j == 0 ? wv + 8 : half);
+      // The next chunk's planes, at different times in the two waves of a SIMD, so that one's VALU work runs beside
+      // the other's MFMAs.
+      if (more && (j == 0) == (wid >= 4)) store(buf ^ 1);
+    }
+    if (wv & 1) {
+      prod(b0, L{}, H{});
+      prod(b0, Mi{}, Mi{});
+      prod(b0, Mi{}, H{});
+    } else {
+      load_a(H{});
+      prod(b0, H{}, L{});
+      prod(b0, H{}, Mi{});
+      prod(b0, H{}, H{});
+    }
+    if (more) load_b(b0, kc + 1, wv);
+  }
+  // The epilogue's inputs, in flight during the exchange of the sums.
+  constexpr int G4 = BN / 4, RPE = PNT / G4, EV = (BM + RPE - 1) / RPE;
+  const int ec4 = tid % G4, er0 = tid / G4, en = n0 + 4 * ec4, enc = min(en, OC - 4);
+  const bool eon = er0 < RPE && en < OC;
+  auto epix = [&](int e) { return min(m0 + min(er0 + e * RPE, BM - 1), M - 1); };
+  floatx4 yres[EV], es, eb;
+  float mkv[EV], rmv[EV];
+  if (o.y && o.accumulate) {
+#pragma unroll
+    for (int e = 0; e < EV; e++) yres[e] = *(const floatx4*)(o.y + (size_t)epix(e) * o.ldy + enc);
+  }
+  if (o.emit.scale) {
+    es = *(const floatx4*)(o.emit.scale + enc);
+    eb = *(const floatx4*)(o.emit.bias + enc);
+#pragma unroll
+    for (int e = 0; e < EV; e++) mkv[e] = o.emit.mask[epix(e)];
+  }
+  if (o.rowmask) {
+#pragma unroll
+    for (int e = 0; e < EV; e++) rmv[e] = o.rowmask[epix(e)];
+  }
+  lds_barrier();  // every wave is done reading the chunks
+
+  float* const Cs = (float*)smem;
+#pragma unroll
+  for (int i = 0; i < WB; i++)
+#pragma unroll
+    for (int j = 0; j < WC; j++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) Cs[(wv * BM + wr + i * 16 + 4 * g4 + r) * LDC + (wc + j) * 16 + r16] = acc[i][j][r];
+  lds_barrier();
+#pragma unroll
+  for (int e = 0; e < EV; e++) {
+    const int row = er0 + e * RPE, m = m0 + row;
+    if (eon && row < BM && m < M) {
+      floatx4 sum = *(const floatx4*)(Cs + row * LDC + 4 * ec4);
+#pragma unroll
+      for (int q = 1; q < 4; q++) sum += *(const floatx4*)(Cs + (q * BM + row) * LDC + 4 * ec4);
+      conv_store4<float, SC >= 0 ? ((SC & SF_EMIT) ? ACT_MISH : ACT_ID) : -1, SC>(o, m, en, sum, yres[e], rmv[e], es, eb,
+                                                                                  mkv[e]);
+    }
+  }
+}
+
+uint16_t bf16_bits(float v) {
+  uint32_t u;
+  v = conv_round_operand(v, PREC_BF16);
+  std::memcpy(&u, &v, 4);
+  return (uint16_t)(u >> 16);
+}
+
+}  // namespace
+
+// w [oc][ic][3][3] -> fragments [16-column block][chunk][step][plane], lane l, element e holding column l % 16, input
+// channel 64 chunk + 32 (step % 2) + 8 (l / 16) + e at tap step / 2; two bf16 per float of `out`, zeros past oc and ic
+// (up to a multiple of 192 columns, so that every tile width reads whole packed blocks).
+void conv_split_pack_weights(const float* w, int oc, int ic, std::vector<float>& out) {
+  const int cbs = round_up(oc, 192) / 16, nch = (ic + PCH - 1) / PCH;
+  std::vector<uint16_t> p((size_t)cbs * nch * PSTEPS * 3 * PFRAG, 0);
+  for (int cb = 0; cb < cbs; cb++)
+    for (int kc = 0; kc < nch; kc++)
+      for (int s = 0; s < PSTEPS; s++)
+        for (int l = 0; l < 64; l++)
+          for (int e = 0; e < 8; e++) {
+            const int col = cb * 16 + l % 16, i = kc * PCH + (s & 1) * 32 + (l / 16) * 8 + e;
+            if (col >= oc || i >= ic) continue;
+            float v = w[((size_t)col * ic + i) * 9 + s / 2];
+            const size_t at = (((size_t)cb * nch + kc) * PSTEPS + s) * 3 * PFRAG + l * 8 + e;
+            for (int q = 0; q < 3; q++) {
+              p[at + q * PFRAG] = bf16_bits(v);
+              v -= conv_round_operand(v, PREC_BF16);
+            }
+          }
+  out.resize(p.size() / 2);
+  std::memcpy(out.data(), p.data(), p.size() * 2);
+}
+
+template <int MB, int NB>
+static void split_launch(const float* x, int ldx, int IC, const bf16* w, int OC, const ConvOut& o, int M, hipStream_t s) {
+  const int ntl = (OC + 16 * NB - 1) / (16 * NB), nch = (IC + PCH - 1) / PCH;
+  const int grid = round_up((M + 16 * MB - 1) / (16 * MB), 8) * ntl;
+  auto go = [&](auto kernel) { launch_k(kernel, grid, PNT, 0, s, x, ldx, IC, w, nch, OC, M, ntl, o); };
+  const int sfl = store_flags(o);
+  switch ((sfl & SF_EMIT) && o.emit.act != ACT_MISH ? -1 : sfl) {  // the store cases of igemm_launch
+    case SF_EMIT: go(conv3_split_kernel<MB, NB, SF_EMIT>); return;
+    case SF_Y: go(conv3_split_kernel<MB, NB, SF_Y>); return;
+    case SF_Y | SF_ACC | SF_EMIT: go(conv3_split_kernel<MB, NB, SF_Y | SF_ACC | SF_EMIT>); return;
+    case SF_Y | SF_ACC | SF_YDEAD | SF_EMIT: go(conv3_split_kernel<MB, NB, SF_Y | SF_ACC | SF_YDEAD | SF_EMIT>); return;
+    default: go(conv3_split_kernel<MB, NB, -1>);
+  }
+}
+
+void launch_conv_split(const float* x, int ldx, int IC, const void* w, int OC, const ConvOut& o, int B, hipStream_t s) {
+  if (IC % 8 || ldx % 4 || OC % 4 || (o.y && o.ldy % 4) || (o.yt && o.ldyt % 4) || (o.colbias && o.ld_colbias % 4) ||
+      (o.emit.scale && o.emit.ld % 4) || ((uintptr_t)x | (uintptr_t)w) % 16 || o.pool.psum)
+    throw std::runtime_error("conv_split: channel counts must be multiples of 8 (inputs) and 4 (outputs)");
+  const int M = B * HW;
+  if (M <= 0) return;
+  // The tile whose rounds of 256 workgroups (one per CU: up to 105 KB of LDS) cost least, a round taking time in
+  // proportion to the tile's 16 x 16 blocks and a fixed part (staging, epilogue) of about six blocks' (measured at 192
+  // input channels: 11.3, 23.5 and 30 us for 6, 18 and 24 blocks).
+  int best = 0;
+  long cost = 0;
+  const int tiles[4][2] = {{6, 4}, {6, 3}, {6, 2}, {3, 2}};
+  for (int k = 0; k < 4; k++) {
+    const int mb = tiles[k][0], nb = tiles[k][1];
+    const long wgs = (long)((M + 16 * mb - 1) / (16 * mb)) * ((OC + 16 * nb - 1) / (16 * nb));
+    const long c = (wgs + 255) / 256 * (mb * nb + 6);
+    if (k == 0 || c < cost) best = k, cost = c;
+  }
+  const bf16* wp = (const bf16*)w;
+  switch (best) {
+    case 0: split_launch<6, 4>(x, ldx, IC, wp, OC, o, M, s); break;
+    case 1: split_launch<6, 3>(x, ldx, IC, wp, OC, o, M, s); break;
+    case 2: split_launch<6, 2>(x, ldx, IC, wp, OC, o, M, s); break;
+    default: split_launch<3, 2>(x, ldx, IC, wp, OC, o, M, s);
+  }
+  KGX_CHECK_LAUNCH();
+}
+
+}  // namespace kgx
