@@ -135,9 +135,17 @@ struct GemmArgs {
   // Activation of the compute-type output alone (ACT_ID or ACT_MISH): out.yt = act(C), as the mish FFN's h.
   int yt_act = ACT_ID;
   QkvEpi qkv;
+  bool split3 = false;   // float GEMM whose Bt is the upload of gemm_split_pack_weights (kgx_split.hip)
   bool vec_epi = false;  // set by launch_gemm: the four-column vector epilogue applies
 };
 void launch_gemm(int prec, const GemmArgs& g, hipStream_t s);
+// Float GEMMs on bf16 matrix cores (kgx_split.hip): whether N columns over K (a q|k|v projection of head dim dq, or 0)
+// fit, the packed weights w [N][K], the rows of the row tile over M rows (row tile r on XCD r mod 8), and the launch
+// with launch_gemm's epilogue `epi`.
+bool gemm_split_fits(int N, int K, int dq);
+void gemm_split_pack_weights(const float* w, int N, int K, std::vector<float>& out);
+int gemm_split_rows(int M, int N);
+void launch_gemm_split(const GemmArgs& g, int epi, hipStream_t s);
 // The rows of the row tile that launch_gemm runs a plain GEMM of these sizes on (row tile r on XCD r mod 8).
 int gemm_row_tile(int prec, int M, int N, int K);
 

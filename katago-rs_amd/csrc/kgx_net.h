@@ -110,6 +110,8 @@ class Net {
   void upload_mm(RowMM& mm, const std::vector<float>& w, const std::vector<float>& b);
   const void* take_upload(size_t bytes);
   const void* upload_t(const std::vector<float>& v);  // converted to the compute type
+  bool gemm_split(int N, int K, int dq) const;
+  const void* upload_gemm(const std::vector<float>& w, int N, int K, int dq);
   size_t tsize() const { return prec_ == PREC_F32 ? 4 : 2; }
 
   // Planning.

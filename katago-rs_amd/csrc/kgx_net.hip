@@ -133,6 +133,16 @@ const void* Net::upload_t(const std::vector<float>& v) {
   return d;
 }
 
+// Whether a GEMM runs as a three-plane product of float operands, and its weights' upload (B^T rows [N][K]).
+bool Net::gemm_split(int N, int K, int dq) const { return conv_mode_ == CONV_SPLIT && gemm_split_fits(N, K, dq); }
+
+const void* Net::upload_gemm(const std::vector<float>& w, int N, int K, int dq) {
+  if (!gemm_split(N, K, dq)) return upload_t(w);
+  std::vector<float> p;
+  gemm_split_pack_weights(w.data(), N, K, p);
+  return upload_f(p);
+}
+
 RowProg Net::row_prog_base() const {
   RowProg p;
   p.mask = mask_;
@@ -421,7 +431,8 @@ std::shared_ptr<ConvOut> Net::emit_conv(const ConvDesc& c, const void* x, int ld
   }
   const int vec = prec == PREC_F32 ? 4 : 8;
   if (c.ky == 1 && c.kx == 1 && !nchw && c.ic % vec == 0 && ldx % vec == 0) {
-    const void* dW = upload_t(c.w);  // [oc][ic] is already the B^T layout
+    const void* dW = upload_gemm(c.w, oc, ic, 0);  // [oc][ic] is already the B^T layout
+    const bool split3 = gemm_split(oc, ic, 0);
     Op gm;
     gm.launch = [=](hipStream_t s, int B) {
       GemmArgs g;
@@ -429,6 +440,7 @@ std::shared_ptr<ConvOut> Net::emit_conv(const ConvDesc& c, const void* x, int ld
       g.Bt = dW; g.ldb = ic;
       g.out = *out;
       g.M = B * HW; g.N = oc; g.K = ic;
+      g.split3 = split3;
       launch_gemm(prec, g, s);
     };
     gm.cls = "gemm_1x1";
@@ -463,10 +475,12 @@ std::shared_ptr<ConvOut> Net::emit_conv(const ConvDesc& c, const void* x, int ld
 std::shared_ptr<ConvOut> Net::emit_token_gemm(const void* A, int lda, const void* Bt, int N, int K, const ConvOut& o,
                                               const char* cls, bool glu, const QkvEpi& qkv, int yt_act) {
   const int prec = prec_;
+  const bool split3 = gemm_split(N, K, qkv.dq);
   auto out = std::make_shared<ConvOut>(o);
   Op op;
   op.launch = [=](hipStream_t s, int B) {
     GemmArgs g;
+    g.split3 = split3;
     g.A = A; g.lda = lda;
     g.Bt = Bt; g.ldb = K;
     g.out = *out;
@@ -511,11 +525,11 @@ void Net::emit_attention(const BlockDesc& b, int depth) {
     for (int k = 0; k < c; k++) w[(size_t)(nq + j) * c + k] = b.k.w[(size_t)k * nk + col_of(j)];
   for (int j = 0; j < nv; j++)
     for (int k = 0; k < c; k++) w[(size_t)(nq + nk + j) * c + k] = b.v.w[(size_t)k * nv + j];
-  const void* dWqkv = upload_t(w);
+  const void* dWqkv = upload_gemm(w, nqkv, c, dq);
   std::vector<float> wo((size_t)c * H * dv);
   for (int o = 0; o < c; o++)
     for (int k = 0; k < H * dv; k++) wo[(size_t)o * H * dv + k] = b.o.w[(size_t)k * c + o];
-  const void* dWo = upload_t(wo);
+  const void* dWo = upload_gemm(wo, c, H * dv, 0);
   // RoPE tables [tables][HW][dq/2], float, as computeRopeCosSin (bin2onnx.py:449-485).
   const float* dcos = nullptr;
   const float* dsin = nullptr;
@@ -612,11 +626,11 @@ void Net::emit_ffn(const BlockDesc& b, int depth) {
       w1[(size_t)row_of(f, false) * c + k] = b.l1.w[(size_t)k * F + f];
       if (b.swiglu) w1[(size_t)row_of(f, true) * c + k] = b.lg.w[(size_t)k * F + f];
     }
-  const void* dW1 = upload_t(w1);
+  const void* dW1 = upload_gemm(w1, Fu, c, 0);
   std::vector<float> w2((size_t)c * F);
   for (int o = 0; o < c; o++)
     for (int f = 0; f < F; f++) w2[(size_t)o * F + f] = b.l2.w[(size_t)f * c + o];
-  const void* dW2 = upload_t(w2);
+  const void* dW2 = upload_gemm(w2, c, F, 0);
   const float* lnw = upload_f(b.ln_w);
   const float eps = b.ln_eps;
   void* nrm = nrm_;

@@ -1,4 +1,4 @@
-// Float 3x3 convolutions on the bf16 matrix cores. Every float operand is split into three bf16 planes, x = h + m + l
+// Float 3x3 convolutions and GEMMs on the bf16 matrix cores. Every float operand is split into three bf16 planes, x = h + m + l
 // (each the rounding of what the planes before it leave: 24 significant bits, float's exponent range), and a product
 // is taken as l h + m m + m h + h l + h m + h h with float accumulation; the terms left out are below 2^-26 of the
 // product. Six v_mfma_f32_16x16x32_bf16 take 96 cycles where v_mfma_f32_16x16x4_f32 takes 256 for the same products,
@@ -16,8 +16,9 @@
 // GEMMs and output transform (F(4x4,3x3)); 128 -> 128 at 8 boards (48 x 32): 9.1 against 37 us. The MFMAs are 12 us of
 // the first; splitting the operands costs 2.5 us of VALU time, the first stage and the epilogue 4.
 // An infinite operand gives NaN where it is read (its second plane is inf - inf).
-#include "kgx_device.h"
+#include "kgx_gemm_epi.h"
 
+#include <climits>
 #include <cstring>
 #include <vector>
 
@@ -271,11 +272,153 @@ __global__ __launch_bounds__(PNT, 1) void conv3_split_kernel(const float* __rest
   }
 }
 
-uint16_t bf16_bits(float v) {
-  uint32_t u;
-  v = conv_round_operand(v, PREC_BF16);
-  std::memcpy(&u, &v, 4);
-  return (uint16_t)(u >> 16);
+// C[M][N] = A[M][K] Bt[N][K]^T with float A split in registers and Bt packed as three planes (fragments [16-column block]
+// [32-channel step][plane]). A workgroup computes 16 MB rows x 64 columns; its four pairs of waves split the K steps
+// (pair w takes w, w + 4, ...), each reading its own fragments of both operands straight from memory, one step ahead:
+// no operand passes through LDS and no barrier stands in the loop, so a product of few tiles (where the latency of
+// its serial K loop sets the time) runs a quarter of the steps one after the other. The pairs' sums are added in
+// order, whatever the tile. The waves of a pair split the rows (MB = 6) or the columns (MB = 2).
+// Against the float matrix unit's 64 x 64 tiles (one 16-channel stage after the other): N = 384 over K = 384 and 1024 at
+// 1083 rows 32.7 -> 12.7 us on average, K = 384 into 2048 gated columns 28.3 -> 21.5; against its 128 x 128 tiles at 3610
+// rows, where both operands' reads from L2 bound it (about 64 bytes a cycle and CU), 149 -> 140 and 76 -> 59 us.
+template <int MB, int EPI>
+__global__ __launch_bounds__(PNT, MB == 2 ? 4 : 2) void gemm_split_kernel(const float* __restrict__ A, const bf16* __restrict__ W, int lda,
+                                                            int M, int N, int K, int ntl, GemmArgs g) {
+  constexpr int BM = 16 * MB, BN = 64, NB = 4;
+  constexpr int WM = MB == 6 ? 2 : 1, WN = 2 / WM, WB = MB / WM, WC = NB / WN;
+  constexpr int ELD = BN + 4;
+  __shared__ __align__(128) float smem[4 * BM * ELD];
+  const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wv = wid & 3, wr = WM == 2 ? (wid >> 2) * WB * 16 : 0, wc = WN == 2 ? (wid >> 2) * WC : 0;
+  const int r16 = lane & 15, g4 = lane >> 4;
+  const int slot = blockIdx.x >> 3, u = slot / ntl, nt = slot - u * ntl, mt = u * 8 + (blockIdx.x & 7);
+  const int m0 = mt * BM, n0 = nt * BN;
+  if (m0 >= M) return;
+
+  const int steps = K / 32;
+  const float* ap[WB];  // this lane's row of each block (rows past M read the last one, never stored)
+#pragma unroll
+  for (int i = 0; i < WB; i++) ap[i] = A + (size_t)min(m0 + wr + i * 16 + r16, M - 1) * lda + g4 * 8;
+  const bf16* const wb = W + (size_t)(nt * NB + wc) * steps * 3 * PFRAG + lane * 8;
+  floatx4 raw[WB][2];
+  bf16x8 a[WB][3], b0[WC][3], b1[WC][3];
+  auto load_a = [&](int s) {
+#pragma unroll
+    for (int i = 0; i < WB; i++) {
+      raw[i][0] = *(const floatx4*)(ap[i] + s * 32);
+      raw[i][1] = *(const floatx4*)(ap[i] + s * 32 + 4);
+    }
+  };
+  auto load_b = [&](bf16x8 (&d)[WC][3], int s) {
+#pragma unroll
+    for (int j = 0; j < WC; j++)
+#pragma unroll
+      for (int q = 0; q < 3; q++) d[j][q] = *(const bf16x8*)(wb + (((size_t)j * steps + s) * 3 + q) * PFRAG);
+  };
+  floatx4 acc[WB][WC];
+#pragma unroll
+  for (int i = 0; i < WB; i++)
+#pragma unroll
+    for (int j = 0; j < WC; j++) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  auto prod = [&](const bf16x8 (&d)[WC][3], auto pa, auto pb) {
+#pragma unroll
+    for (int i = 0; i < WB; i++)
+#pragma unroll
+      for (int j = 0; j < WC; j++)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i][decltype(pa)::value], d[j][decltype(pb)::value],
+                                                            acc[i][j], 0, 0, 0);
+  };
+  typedef std::integral_constant<int, 0> H;
+  typedef std::integral_constant<int, 1> Mi;
+  typedef std::integral_constant<int, 2> L;
+  auto step = [&](const bf16x8 (&d)[WC][3], bf16x8 (&dn)[WC][3], int s) {
+#pragma unroll
+    for (int i = 0; i < WB; i++) {
+      u32x4 p[3];
+      split3(raw[i], p);
+#pragma unroll
+      for (int q = 0; q < 3; q++) a[i][q] = __builtin_bit_cast(bf16x8, p[q]);
+    }
+    const int sn = min(s + 4, steps - 1);
+    load_a(sn);
+    load_b(dn, sn);
+    __builtin_amdgcn_sched_barrier(0);
+    prod(d, L{}, H{});
+    prod(d, Mi{}, Mi{});
+    prod(d, Mi{}, H{});
+    prod(d, H{}, L{});
+    prod(d, H{}, Mi{});
+    prod(d, H{}, H{});
+  };
+  load_a(min(wv, steps - 1));
+  load_b(b0, min(wv, steps - 1));
+#pragma unroll 1
+  for (int s = wv; s < steps; s += 8) {
+    step(b0, b1, s);
+    if (s + 4 < steps) step(b1, b0, s + 4);
+  }
+
+  // The inputs of the epilogues that read memory, in flight during the exchange of the sums: thread tid finishes
+  // columns 4 (tid % 16) .. + 3 of rows tid / 16 + 32 v (clamped indices; the stores skip what lies outside).
+  constexpr int EV = BM * 16 / PNT;
+  constexpr bool OWN = EPI == EPI_GEN || EPI == EPI_ACC;
+  const ConvOut& o = g.out;
+  const int en = n0 + (tid & 15) * 4, enc = min(en, N - 4);
+  floatx4 yres[EV], es = {1.f, 1.f, 1.f, 1.f}, eb = {0.f, 0.f, 0.f, 0.f};
+  float rmv[EV], mkv[EV];
+  if constexpr (OWN) {
+    if (EPI == EPI_GEN && o.emit.scale) {
+      es = *(const floatx4*)(o.emit.scale + enc);
+      eb = *(const floatx4*)(o.emit.bias + enc);
+    }
+#pragma unroll
+    for (int v = 0; v < EV; v++) {
+      const int m = min(m0 + (tid >> 4) + 32 * v, M - 1);
+      yres[v] = o.y && o.accumulate ? *(const floatx4*)(o.y + (size_t)m * o.ldy + enc) : floatx4{0.f, 0.f, 0.f, 0.f};
+      rmv[v] = o.rowmask ? o.rowmask[m] : 1.f;
+      mkv[v] = EPI == EPI_GEN && o.emit.scale ? o.emit.mask[m] : 1.f;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < WB; i++)
+#pragma unroll
+    for (int j = 0; j < WC; j++)
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+        smem[(wv * BM + wr + i * 16 + 4 * g4 + r) * ELD + (wc + j) * 16 + r16] = acc[i][j][r];
+  lds_barrier();
+#pragma unroll
+  for (int v = 0; v < EV; v++) {
+    const int e = tid + PNT * v, m = m0 + (e >> 4);
+    float* p = smem + (e >> 4) * ELD + (e & 15) * 4;
+    floatx4 sum = *(const floatx4*)p;
+#pragma unroll
+    for (int q = 1; q < 4; q++) sum += *(const floatx4*)(p + q * BM * ELD);
+    if constexpr (!OWN) {
+      *(floatx4*)p = sum;
+    } else if (m < M && en < N) {
+      if constexpr (EPI == EPI_ACC) *(floatx4*)(o.y + (size_t)m * o.ldy + en) = sum * rmv[v] + yres[v];
+      else conv_store4<float>(o, m, en, sum, yres[v], rmv[v], es, eb, mkv[v]);
+    }
+  }
+  if constexpr (!OWN) {
+    lds_barrier();
+    gemm_tile_epilogue<float, EPI, BM, BN, PNT>(smem, g, o, m0, n0, M, N, tid);
+  }
+}
+
+// The three planes of v (round to nearest even; infinities and NaN keep their first plane).
+inline void host_split3(float v, uint16_t* p, size_t plane) {
+  for (int q = 0; q < 3; q++) {
+    uint32_t u;
+    std::memcpy(&u, &v, 4);
+    if ((u & 0x7f800000u) != 0x7f800000u) u += 0x7fffu + ((u >> 16) & 1u);
+    u &= 0xffff0000u;
+    p[q * plane] = (uint16_t)(u >> 16);
+    float h;
+    std::memcpy(&h, &u, 4);
+    v -= h;
+  }
 }
 
 }  // namespace
@@ -293,12 +436,8 @@ void conv_split_pack_weights(const float* w, int oc, int ic, std::vector<float>&
           for (int e = 0; e < 8; e++) {
             const int col = cb * 16 + l % 16, i = kc * PCH + (s & 1) * 32 + (l / 16) * 8 + e;
             if (col >= oc || i >= ic) continue;
-            float v = w[((size_t)col * ic + i) * 9 + s / 2];
-            const size_t at = (((size_t)cb * nch + kc) * PSTEPS + s) * 3 * PFRAG + l * 8 + e;
-            for (int q = 0; q < 3; q++) {
-              p[at + q * PFRAG] = bf16_bits(v);
-              v -= conv_round_operand(v, PREC_BF16);
-            }
+            host_split3(w[((size_t)col * ic + i) * 9 + s / 2],
+                        p.data() + (((size_t)cb * nch + kc) * PSTEPS + s) * 3 * PFRAG + l * 8 + e, PFRAG);
           }
   out.resize(p.size() / 2);
   std::memcpy(out.data(), p.data(), p.size() * 2);
@@ -345,6 +484,56 @@ void launch_conv_split(const float* x, int ldx, int IC, const void* w, int OC, c
     default: split_launch<3, 2>(x, ldx, IC, wp, OC, o, M, s);
   }
   KGX_CHECK_LAUNCH();
+}
+
+bool gemm_split_fits(int N, int K, int dq) { return K % 32 == 0 && N % 4 == 0 && (dq == 0 || 64 % dq == 0); }
+
+// w [N][K] -> fragments [16-column block][step][plane], lane l, element e holding column l % 16, input 32 step +
+// 8 (l / 16) + e; two bf16 per float of `out`, zeros past N up to a multiple of 64 columns.
+void gemm_split_pack_weights(const float* w, int N, int K, std::vector<float>& out) {
+  const int cbs = round_up(N, 64) / 16, steps = K / 32;
+  std::vector<uint16_t> p((size_t)cbs * steps * 3 * PFRAG, 0);
+  for (int cb = 0; cb < cbs; cb++)
+    for (int s = 0; s < steps; s++)
+      for (int l = 0; l < 64; l++)
+        for (int e = 0; e < 8; e++) {
+          const int col = cb * 16 + l % 16;
+          if (col >= N) continue;
+          host_split3(w[(size_t)col * K + s * 32 + (l / 16) * 8 + e],
+                      p.data() + ((size_t)cb * steps + s) * 3 * PFRAG + l * 8 + e, PFRAG);
+        }
+  out.resize(p.size() / 2);
+  std::memcpy(out.data(), p.data(), p.size() * 2);
+}
+
+// 96-row tiles (one workgroup per CU), or 32-row tiles (two) where their rounds cost less (a round: the 16 x 16 blocks
+// of a CU's workgroups and a fixed part of about eight blocks' time).
+int gemm_split_rows(int M, int N) {
+  const long nt = (N + 63) / 64, wide = (M + 95) / 96 * nt, small = (M + 31) / 32 * nt;
+  return (wide + 255) / 256 * (24 + 8) <= (small + 511) / 512 * (16 + 8) ? 96 : 32;
+}
+
+template <int MB>
+static void gemm_split_launch(const GemmArgs& g, int epi, hipStream_t s) {
+  const int ntl = (g.N + 63) / 64, grid = round_up((g.M + 16 * MB - 1) / (16 * MB), 8) * ntl;
+  auto go = [&](auto kernel) {
+    launch_k(kernel, grid, PNT, 0, s, (const float*)g.A, (const bf16*)g.Bt, (int)g.lda, g.M, g.N, g.K, ntl, g);
+  };
+  switch (epi) {
+    case EPI_YT: go(gemm_split_kernel<MB, EPI_YT>); break;
+    case EPI_ACC: go(gemm_split_kernel<MB, EPI_ACC>); break;
+    case EPI_GLU: go(gemm_split_kernel<MB, EPI_GLU>); break;
+    case EPI_QKV: go(gemm_split_kernel<MB, EPI_QKV>); break;
+    case EPI_YTMISH: go(gemm_split_kernel<MB, EPI_YTMISH>); break;
+    default: go(gemm_split_kernel<MB, EPI_GEN>);
+  }
+}
+
+void launch_gemm_split(const GemmArgs& g, int epi, hipStream_t s) {
+  if (!gemm_split_fits(g.N, g.K, g.qkv.dq) || g.lda % 4 || g.lda > INT_MAX || ((uintptr_t)g.A | (uintptr_t)g.Bt) % 16)
+    throw std::runtime_error("gemm: shape or alignment does not fit the three-plane product");
+  if (gemm_split_rows(g.M, g.N) == 96) gemm_split_launch<6>(g, epi, s);
+  else gemm_split_launch<2>(g, epi, s);
 }
 
 }  // namespace kgx
