@@ -52,8 +52,8 @@ template <int MB, int NB, int SC>
 __global__ __launch_bounds__(PNT, 1) void conv3_split_kernel(const float* __restrict__ X, int ldx, int IC,
                                                              const bf16* __restrict__ W, int nch, int OC, int M, int ntl,
                                                              ConvOut o) {
-  // Two waves per step share: over the rows, or over the columns of the tile that is too wide or too short for that.
-  constexpr int WM = MB == 6 && NB < 4 ? 2 : 1, WN = 2 / WM, WB = MB / WM, WC = NB / WN;
+  // Two waves per step share: over the rows, or over the columns of the tile that is too short for that.
+  constexpr int WM = MB == 6 ? 2 : 1, WN = 2 / WM, WB = MB / WM, WC = NB / WN;
   constexpr int BM = 16 * MB, BN = 16 * NB, AR = BM + 2 * PHALO;
   constexpr int PLB = (AR + 1) * 128, BUF = 3 * PLB;  // bytes of a chunk's plane (its last row zero) and of a chunk
   constexpr int LDC = BN + 4, CB = 4 * BM * LDC * 4;
