@@ -144,7 +144,7 @@ void launch_gemm(int prec, const GemmArgs& g, hipStream_t s);
 // with launch_gemm's epilogue `epi`.
 bool gemm_split_fits(int N, int K, int dq);
 void gemm_split_pack_weights(const float* w, int N, int K, std::vector<float>& out);
-int gemm_split_rows(int M, int N);
+int gemm_split_rows(int M, int N, int K);
 void launch_gemm_split(const GemmArgs& g, int epi, hipStream_t s);
 // The rows of the row tile that launch_gemm runs a plain GEMM of these sizes on (row tile r on XCD r mod 8).
 int gemm_row_tile(int prec, int M, int N, int K);

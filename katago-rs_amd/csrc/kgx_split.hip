@@ -278,9 +278,9 @@ __global__ __launch_bounds__(PNT, 1) void conv3_split_kernel(const float* __rest
 // no operand passes through LDS and no barrier stands in the loop, so a product of few tiles (where the latency of
 // its serial K loop sets the time) runs a quarter of the steps one after the other. The pairs' sums are added in
 // order, whatever the tile. The waves of a pair split the rows (MB = 6) or the columns (MB = 2).
-// Against the float matrix unit's 64 x 64 tiles (one 16-channel stage after the other): N = 384 over K = 384 and 1024 at
-// 1083 rows 32.7 -> 12.7 us on average, K = 384 into 2048 gated columns 28.3 -> 21.5; against its 128 x 128 tiles at 3610
-// rows, where both operands' reads from L2 bound it (about 64 bytes a cycle and CU), 149 -> 140 and 76 -> 59 us.
+// Against the float matrix unit's 64 x 64 tiles (one 16-channel stage after the other): N = 384 over K = 384 and 1536 at
+// 1083 rows 32.7 -> 12.7 us on average, K = 384 into 1536 columns 28.3 -> 21.5; against its 128 x 128 tiles at 3610
+// rows, where both operands' reads from L2 bound it (about 64 bytes a cycle and CU), 149 -> 140 and 76 -> 59 us (gemm_split_lds_kernel takes those).
 template <int MB, int EPI>
 __global__ __launch_bounds__(PNT, MB == 2 ? 4 : 2) void gemm_split_kernel(const float* __restrict__ A, const bf16* __restrict__ W, int lda,
                                                             int M, int N, int K, int ntl, GemmArgs g) {
@@ -407,6 +407,157 @@ __global__ __launch_bounds__(PNT, MB == 2 ? 4 : 2) void gemm_split_kernel(const 
   }
 }
 
+// The same product on 128 x 128 tiles with both operands' planes in LDS, for grids that fill the chip: eight waves of
+// 64 x 32 share each 32-channel step's fragments (A split on its way, one task of 8 channels per thread; the packed
+// weights straight into LDS), double-buffered with one barrier per step, so an operand byte read from L2 feeds twice to
+// four times the MFMAs. The steps run in the order of the wave pairs' shares (0, 4, 8, ..., 1, 5, ...) and each
+// share's sum is added to the total when it ends: the sums of gemm_split_kernel, in its order. The next step's A values
+// were loaded a whole step before they are split, between this step's products. 3610 rows x 4096 columns over K = 512:
+// 140 -> 99 us against the 96 x 64 tile (149 on the float matrix unit), 1536 columns 59 -> 51; bound by the barrier per
+// step (the MFMAs are 40 us of the 99).
+template <int EPI>
+__global__ __launch_bounds__(PNT, 2) void gemm_split_lds_kernel(const float* __restrict__ A, const bf16* __restrict__ W,
+                                                                int lda, int M, int N, int K, int ntl, GemmArgs g) {
+  constexpr int BM = 128, BN = 128, WB = 4, WC = 2, ELD = BN + 4;
+  constexpr int AB = BM / 16 * 3 * 1024, BUF = AB + BN / 16 * 3 * 1024;  // bytes of a step's A planes, of a step
+  static_assert(BM * ELD * 4 <= 2 * BUF, "the float tile reuses the steps");
+  __shared__ __align__(1024) char smem[2 * BUF];
+  const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wid >> 2, wn = wid & 3, r16 = lane & 15, g4 = lane >> 4;
+  const int slot = blockIdx.x >> 3, u = slot / ntl, nt = slot - u * ntl, mt = u * 8 + (blockIdx.x & 7);
+  const int m0 = mt * BM, n0 = nt * BN;
+  if (m0 >= M) return;
+
+  const int steps = K / 32;
+  // Staging of A: thread tid takes channels 8 (tid % 4) .. + 7 of row tid / 4 (rows past M read the last one) into
+  // fragment order: [16-row block][plane][lane][16 bytes].
+  const int srow = tid >> 2, sch = tid & 3;
+  const float* const ap = A + (size_t)min(m0 + srow, M - 1) * lda + sch * 8;
+  char* const ad = smem + (srow >> 4) * 3072 + (sch * 16 + (srow & 15)) * 16;
+  floatx4 raw[2], nxt[2];  // the next step's values, and the ones after
+  auto load_a = [&](floatx4 (&d)[2], int s) {
+    d[0] = *(const floatx4*)(ap + s * 32);
+    d[1] = *(const floatx4*)(ap + s * 32 + 4);
+  };
+  auto store_a = [&](int buf) {
+    u32x4 p[3];
+    asm volatile("" : "+v"(raw[0]), "+v"(raw[1]));  // (split here, not where the values arrive)
+    split3(raw, p);
+#pragma unroll
+    for (int q = 0; q < 3; q++) *(u32x4*)(ad + buf * BUF + q * 1024) = p[q];
+  };
+  // Wave wid's column block of the packed weights (blocks past the packed ones lie outside the range and read as zero).
+  const int cb = n0 / 16 + wid, wbytes = (N + 63) / 64 * 4 * steps * 3 * 1024;
+  auto dma_b = [&](int buf, int s) {
+#pragma unroll
+    for (int q = 0; q < 3; q++)
+      lds_load16(W, wbytes, smem + buf * BUF + AB + (wid * 3 + q) * 1024, ((cb * steps + s) * 3 + q) * 1024 + lane * 16);
+  };
+  floatx4 acc[WB][WC], tot[WB][WC];
+#pragma unroll
+  for (int i = 0; i < WB; i++)
+#pragma unroll
+    for (int j = 0; j < WC; j++) acc[i][j] = tot[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  auto after = [&](int s) { return s + 4 < steps ? s + 4 : (s & 3) + 1; };  // the step after s (4: past the last)
+
+  load_a(raw, 0);
+  dma_b(0, 0);
+  store_a(0);
+  int s1 = after(0);
+  load_a(raw, s1);  // (at least four steps: the launch)
+#pragma unroll 1
+  for (int t = 0, s = 0; t < steps; t++, s = s1, s1 = after(s1)) {
+    const int buf = t & 1;
+    // (The direct loads are not counted by the compiler.)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (t + 1 < steps) {
+      dma_b(buf ^ 1, s1);
+      load_a(nxt, t + 2 < steps ? after(s1) : s1);
+    }
+    bf16x8 a[WB][3], b[WC][3];
+    const char* const as = smem + buf * BUF + wm * WB * 3072 + lane * 16;
+    const char* const bs = smem + buf * BUF + AB + wn * WC * 3072 + lane * 16;
+#pragma unroll
+    for (int q = 2; q >= 0; q--) {
+#pragma unroll
+      for (int i = 0; i < WB; i++) a[i][q] = *(const bf16x8*)(as + i * 3072 + q * 1024);
+#pragma unroll
+      for (int j = 0; j < WC; j++) b[j][2 - q] = *(const bf16x8*)(bs + j * 3072 + (2 - q) * 1024);
+    }
+    auto prod = [&](int pa, int pb) {
+#pragma unroll
+      for (int i = 0; i < WB; i++)
+#pragma unroll
+        for (int j = 0; j < WC; j++)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i][pa], b[j][pb], acc[i][j], 0, 0, 0);
+    };
+    prod(2, 0);
+    prod(1, 1);
+    prod(1, 0);
+    if (t + 1 < steps) {
+      store_a(buf ^ 1);
+      raw[0] = nxt[0];
+      raw[1] = nxt[1];
+    }
+    prod(0, 2);
+    prod(0, 1);
+    prod(0, 0);
+    if (s + 4 >= steps) {  // the share's last step
+#pragma unroll
+      for (int i = 0; i < WB; i++)
+#pragma unroll
+        for (int j = 0; j < WC; j++) {
+          tot[i][j] += acc[i][j];
+          acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+  }
+
+  constexpr int EV = BM * (BN / 4) / PNT;
+  constexpr bool OWN = EPI == EPI_GEN || EPI == EPI_ACC;
+  const ConvOut& o = g.out;
+  const int en = n0 + (tid & 31) * 4, enc = min(en, N - 4);
+  floatx4 yres[EV], es = {1.f, 1.f, 1.f, 1.f}, eb = {0.f, 0.f, 0.f, 0.f};
+  float rmv[EV], mkv[EV];
+  if constexpr (OWN) {  // (as gemm_split_kernel's)
+    if (EPI == EPI_GEN && o.emit.scale) {
+      es = *(const floatx4*)(o.emit.scale + enc);
+      eb = *(const floatx4*)(o.emit.bias + enc);
+    }
+#pragma unroll
+    for (int v = 0; v < EV; v++) {
+      const int m = min(m0 + (tid >> 5) + 16 * v, M - 1);
+      yres[v] = o.y && o.accumulate ? *(const floatx4*)(o.y + (size_t)m * o.ldy + enc) : floatx4{0.f, 0.f, 0.f, 0.f};
+      rmv[v] = o.rowmask ? o.rowmask[m] : 1.f;
+      mkv[v] = EPI == EPI_GEN && o.emit.scale ? o.emit.mask[m] : 1.f;
+    }
+  }
+  lds_barrier();  // every wave is done reading the steps
+  float* const Et = (float*)smem;
+#pragma unroll
+  for (int i = 0; i < WB; i++)
+#pragma unroll
+    for (int j = 0; j < WC; j++)
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+        Et[((wm * WB + i) * 16 + 4 * g4 + r) * ELD + (wn * WC + j) * 16 + r16] = tot[i][j][r];
+  lds_barrier();
+  if constexpr (!OWN) {
+    gemm_tile_epilogue<float, EPI, BM, BN, PNT>(Et, g, o, m0, n0, M, N, tid);
+  } else {
+#pragma unroll
+    for (int v = 0; v < EV; v++) {
+      const int row = (tid >> 5) + 16 * v, m = m0 + row;
+      if (m < M && en < N) {
+        const floatx4 sum = *(const floatx4*)(Et + row * ELD + (tid & 31) * 4);
+        if constexpr (EPI == EPI_ACC) *(floatx4*)(o.y + (size_t)m * o.ldy + en) = sum * rmv[v] + yres[v];
+        else conv_store4<float>(o, m, en, sum, yres[v], rmv[v], es, eb, mkv[v]);
+      }
+    }
+  }
+}
+
 // The three planes of v (round to nearest even; infinities and NaN keep their first plane).
 inline void host_split3(float v, uint16_t* p, size_t plane) {
   for (int q = 0; q < 3; q++) {
@@ -506,34 +657,53 @@ void gemm_split_pack_weights(const float* w, int N, int K, std::vector<float>& o
   std::memcpy(out.data(), p.data(), p.size() * 2);
 }
 
-// 96-row tiles (one workgroup per CU), or 32-row tiles (two) where their rounds cost less (a round: the 16 x 16 blocks
-// of a CU's workgroups and a fixed part of about eight blocks' time).
-int gemm_split_rows(int M, int N) {
-  const long nt = (N + 63) / 64, wide = (M + 95) / 96 * nt, small = (M + 31) / 32 * nt;
-  return (wide + 255) / 256 * (24 + 8) <= (small + 511) / 512 * (16 + 8) ? 96 : 32;
+// The row tile (32 x 64, 96 x 64 or, with at least four steps, 128 x 128 in LDS) whose rounds take least, by times in
+// us of a round of one workgroup per CU (two of the 32-row tile) fitted to measurements: 96 x 64 over 16 steps 14.0 a
+// round (10 rounds at 3610 rows x 4096 columns), 128 x 128 24.8 (4 rounds of the same) and 19.6 over 12 steps (1083 x
+// 1536), 32 x 64 8 and 17 over 12 and 48 steps in one round of one workgroup per CU, 59 over 16 and 64 steps on
+// average in two rounds of two (3610 x 512).
+int gemm_split_rows(int M, int N, int K) {
+  const int steps = K / 32;
+  auto wgs = [&](int rows, int cols) { return (long)((M + rows - 1) / rows) * ((N + cols - 1) / cols); };
+  const long w32 = wgs(32, 64), w96 = wgs(96, 64), w128 = wgs(128, 128);
+  const double t32 = w32 <= 256 ? 0.26 * steps + 5 : (w32 + 511) / 512 * (0.65 * steps + 5);
+  const double t96 = (w96 + 255) / 256 * (0.6 * steps + 4), t128 = (w128 + 255) / 256 * (1.2 * steps + 5);
+  // (Its weights' offsets are 32-bit.)
+  if (steps >= 4 && t128 < t96 && t128 < t32 && 6.0 * (N + 64) * K < INT_MAX) return 128;
+  return t96 <= t32 ? 96 : 32;
+}
+
+template <int MB, int EPI>
+static auto gemm_split_pick() {
+  if constexpr (MB == 8) return gemm_split_lds_kernel<EPI>;
+  else return gemm_split_kernel<MB, EPI>;
 }
 
 template <int MB>
 static void gemm_split_launch(const GemmArgs& g, int epi, hipStream_t s) {
-  const int ntl = (g.N + 63) / 64, grid = round_up((g.M + 16 * MB - 1) / (16 * MB), 8) * ntl;
+  constexpr int BN = MB == 8 ? 128 : 64;
+  const int ntl = (g.N + BN - 1) / BN, grid = round_up((g.M + 16 * MB - 1) / (16 * MB), 8) * ntl;
   auto go = [&](auto kernel) {
     launch_k(kernel, grid, PNT, 0, s, (const float*)g.A, (const bf16*)g.Bt, (int)g.lda, g.M, g.N, g.K, ntl, g);
   };
   switch (epi) {
-    case EPI_YT: go(gemm_split_kernel<MB, EPI_YT>); break;
-    case EPI_ACC: go(gemm_split_kernel<MB, EPI_ACC>); break;
-    case EPI_GLU: go(gemm_split_kernel<MB, EPI_GLU>); break;
-    case EPI_QKV: go(gemm_split_kernel<MB, EPI_QKV>); break;
-    case EPI_YTMISH: go(gemm_split_kernel<MB, EPI_YTMISH>); break;
-    default: go(gemm_split_kernel<MB, EPI_GEN>);
+    case EPI_YT: go(gemm_split_pick<MB, EPI_YT>()); break;
+    case EPI_ACC: go(gemm_split_pick<MB, EPI_ACC>()); break;
+    case EPI_GLU: go(gemm_split_pick<MB, EPI_GLU>()); break;
+    case EPI_QKV: go(gemm_split_pick<MB, EPI_QKV>()); break;
+    case EPI_YTMISH: go(gemm_split_pick<MB, EPI_YTMISH>()); break;
+    default: go(gemm_split_pick<MB, EPI_GEN>());
   }
 }
 
 void launch_gemm_split(const GemmArgs& g, int epi, hipStream_t s) {
   if (!gemm_split_fits(g.N, g.K, g.qkv.dq) || g.lda % 4 || g.lda > INT_MAX || ((uintptr_t)g.A | (uintptr_t)g.Bt) % 16)
     throw std::runtime_error("gemm: shape or alignment does not fit the three-plane product");
-  if (gemm_split_rows(g.M, g.N) == 96) gemm_split_launch<6>(g, epi, s);
-  else gemm_split_launch<2>(g, epi, s);
+  switch (gemm_split_rows(g.M, g.N, g.K)) {
+    case 128: gemm_split_launch<8>(g, epi, s); break;
+    case 96: gemm_split_launch<6>(g, epi, s); break;
+    default: gemm_split_launch<2>(g, epi, s);
+  }
 }
 
 }  // namespace kgx
