@@ -275,7 +275,9 @@ int kg_featurize_rows(int device, int n, const kg_position* rows, int nn_x_len, 
  * in the reference (its convolutions are cubecl kernels with their own tiling, crates/katago-nn-burn/src/wino/
  * kernels.rs); these call the same functions as the kernel and its launcher, and launch nothing.
  * kg_conv_geometry: the configuration that a ks x ks convolution of ic -> oc channels (split: split operands, 1x1
- * only) over `pixels` pixels (batch x 361) runs. */
+ * only) over `pixels` pixels (batch x 361) runs on the large tiles. (A 3x3 of whole 64-channel stages, up to 192 inputs and
+ * outputs, over few pixels, as one board to eleven at 192 outputs, runs conv_small_kernel instead, whose workgroup g
+ * takes pixel tile g / column tiles and column tile g mod column tiles of 64, 128 or 192 pixels x 16 channels.) */
 typedef struct {
   int grid;                /* workgroups launched */
   int threads;             /* threads per workgroup */
@@ -300,7 +302,8 @@ int kg_conv_weight_load(int ks, int ic, int oc, int split, int q, int wave, int 
 int kg_conv_weight_chunk(int row, int chunk);
 /* The nested-bottleneck junction launch (one block's exit 1x1 convolution, 192 -> 384, and the next block's entry
  * 1x1, 384 -> 192, in one kernel) over `pixels` pixels: its workgroup count, and the 48-pixel tile that workgroup
- * `workgroup` computes (-1 when it exits at once). No counterpart in the reference: the index map its kernel uses,
+ * `workgroup` computes (-1 when it exits at once). (Up to 8192 pixels the launch takes 16- or 32-pixel tiles in order
+ * instead, workgroup g tile g.) No counterpart in the reference: the index map its kernel uses,
  * for host-side checks. */
 int kg_junction_tile_of(int pixels, int workgroup, int* grid, int* tile);
 /* The gpool blocks' tile launch (a global-pooling block's mid activation per 192-pixel tile: pooled features,
