@@ -364,7 +364,11 @@ std::shared_ptr<ConvOut> Net::emit_conv(const ConvDesc& c, const void* x, int ld
     ops_.push_back(op);
     return out;
   }
-  if (k3 && conv_mode_ == CONV_SPLIT && !nchw && c.ic % 8 == 0 && ldx % 4 == 0 && c.oc % 4 == 0 &&
+  // Up to 256 x 256 channels the direct split sum, beyond them F(4x4,3x3), whose quarter of the products then outweighs its
+  // transforms: residual nets at f32 against Winograd, 256 channels 1.31x at 32 boards and 1.04x at 128 (192 and 128
+  // 1.2-2.9x over their range), 384 channels 0.98x and 0.88x, 512 channels 0.86x at 64. Not by batch: a row's result
+  // must not depend on it.
+  if (k3 && conv_mode_ == CONV_SPLIT && (long)c.ic * c.oc <= 256 * 256 && !nchw && c.ic % 8 == 0 && ldx % 4 == 0 && c.oc % 4 == 0 &&
       (!o.y || o.ldy % 4 == 0) && (!o.yt || o.ldyt % 4 == 0) && (!o.colbias || o.ld_colbias % 4 == 0) && !o.pool.psum) {
     std::vector<float> w;
     conv_split_pack_weights(c.w.data(), c.oc, c.ic, w);

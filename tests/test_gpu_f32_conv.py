@@ -1,4 +1,4 @@
-"""Float 3x3 convolutions on three-plane bf16 splits (conv3_split_kernel), over channel counts that end inside a 64-channel
+"""Float 3x3 convolutions on three-plane bf16 splits (conv3_split_kernel; beyond 256 x 256 channels Winograd), over channel counts that end inside a 64-channel
 chunk and inside a column tile, and over the batches where the tile changes: against the oracle, and every row equal to
 the same row in another batch; magnitudes far from one, where the planes' exponents range."""
 import numpy as np
@@ -8,7 +8,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("trunk,mid,act,scale", [
-    (192, 192, "ACTIVATION_MISH", 1.0), (128, 72, "ACTIVATION_RELU", 1.0), (40, 264, "ACTIVATION_MISH", 1.0),
+    (192, 192, "ACTIVATION_MISH", 1.0), (128, 72, "ACTIVATION_RELU", 1.0), (40, 264, "ACTIVATION_MISH", 1.0), (256, 264, "ACTIVATION_MISH", 1.0),
     (64, 64, "ACTIVATION_RELU", 1e12), (64, 64, "ACTIVATION_RELU", 1e-12)])
 def test_float_convolutions_match_oracle_in_every_tile(kgx, synth, oracle, trunk, mid, act, scale):
     arch = synth.Arch(f"t-split{mid}", 14, trunk, [("res", mid), ("gpool", trunk, 64), ("res", mid)], mid_c=mid, gpool_c=64,
