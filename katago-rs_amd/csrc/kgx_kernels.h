@@ -171,7 +171,8 @@ const char* conv_igemm_class(int ks, int ic, int oc, bool split = false);
 // per tile (BN) when its kernel computes pooling partials (3x3 with 64-channel column tiles, 192 pixels), else 0.
 int conv_igemm_tile_rows(int ks, int ic, int oc, bool split = false);
 int conv_igemm_pool_cols(int ks, int ic, int oc);
-// The launch geometry of the convolution of these shapes over M pixels, and the index maps its kernel uses (the
+// The launch geometry of the convolution of these shapes over M pixels on the large tiles (launch_conv_igemm runs few
+// pixels on conv_small_mb's), and the index maps its kernel uses (the
 // same functions): workgroup -> (pixel tile, column tile), -1 for a workgroup that exits at once; with the weights
 // straight into LDS, the weight row and chunk that direct load q of (wave, lane) reads and the LDS row and chunk it
 // fills (-1: the spare area), and the stored chunk of a row's logical chunk.
@@ -215,7 +216,7 @@ constexpr int kJunctionInner = 192, kJunctionOuter = 384, kJunctionHead = 96;
 void junction_pack_weights(const float* w_exit, const float* w_entry, int entry_oc, int prec, std::vector<float>& out);
 void launch_junction(int prec, const void* x, const void* x_lo, int ldx, const void* w, const ConvOut& exit_o,
                      const ConvOut& entry_o, int entry_oc, int B, hipStream_t s);
-// The launch's grid over M pixels, and the 48-pixel tile workgroup g computes (tiles past M exit at once).
+// The 48-pixel launch's grid over M pixels (above 8192; fewer take smaller tiles), and the tile workgroup g computes (tiles past M exit at once).
 int junction_grid(int M);
 // The stem junction: the network's stem, a 3x3 convolution of the packed input rows (ldx <= 32 channels, one 16-bit
 // plane) into the trunk with its row bias (eo: y stored, colbias, the emission of the entry's activation), and the

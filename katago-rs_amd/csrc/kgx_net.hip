@@ -288,9 +288,10 @@ void Net::scan(const std::vector<BlockDesc>& blocks, int c, int depth) {
   }
 }
 
-// conv(x) into `o`. 3x3 undilated convs run as Winograd (crates/katago-nn-burn/src/wino/ext.rs:324-437): with
+// conv(x) into `o`. 3x3 undilated convs run as implicit GEMMs (16-bit operands), as the direct sum of three-plane splits
+// (float operands, up to 256 x 256 channels), or as Winograd (crates/katago-nn-burn/src/wino/ext.rs:324-437): with
 // F(2x2,3x3) as an input transform plus one kernel for the 16 point GEMMs and the output transform, with
-// F(4x4,3x3) as input transform, 36 batched MFMA GEMMs and output transform. 1x1 convs over NHWC rows are one MFMA
+// F(4x4,3x3) as input transform, 36 batched MFMA GEMMs and output transform. Float 1x1 convs over NHWC rows are one MFMA
 // GEMM (wino/ext.rs:278-321); anything else is a direct convolution.
 bool Net::igemm_eligible(const ConvDesc& c, bool nchw, int ldx, const ConvOut& o) const {
   const bool k3 = c.ky == 3 && c.kx == 3 && c.dy == 1 && c.dx == 1, k1 = c.ky == 1 && c.kx == 1;

@@ -280,7 +280,8 @@ __global__ __launch_bounds__(PNT, 1) void conv3_split_kernel(const float* __rest
 // order, whatever the tile. The waves of a pair split the rows (MB = 6) or the columns (MB = 2).
 // Against the float matrix unit's 64 x 64 tiles (one 16-channel stage after the other): N = 384 over K = 384 and 1536 at
 // 1083 rows 32.7 -> 12.7 us on average, K = 384 into 1536 columns 28.3 -> 21.5; against its 128 x 128 tiles at 3610
-// rows, where both operands' reads from L2 bound it (about 64 bytes a cycle and CU), 149 -> 140 and 76 -> 59 us (gemm_split_lds_kernel takes those).
+// rows, where both operands' reads from L2 bound it (about 64 bytes a cycle and CU), 149 -> 140 and 76 -> 59 us
+// (gemm_split_lds_kernel takes those).
 template <int MB, int EPI>
 __global__ __launch_bounds__(PNT, MB == 2 ? 4 : 2) void gemm_split_kernel(const float* __restrict__ A, const bf16* __restrict__ W, int lda,
                                                             int M, int N, int K, int ntl, GemmArgs g) {
