@@ -15,9 +15,14 @@
 // 192 -> 192 channels at 16 boards (96 x 48 tiles, 244 workgroups): 23.5 us, against 53 us of input transform, 36 point
 // GEMMs and output transform (F(4x4,3x3)); 128 -> 128 at 8 boards (48 x 32): 9.1 against 37 us. The MFMAs are 12 us of
 // the first; splitting the operands costs 2.5 us of VALU time, the first stage and the epilogue 4.
-// An infinite operand gives NaN where it is read (its second plane is inf - inf).
+// An activation that is infinite, or rounds to infinity as a bf16 (from 3.3962e38), has no planes (inf - inf). A GEMM's
+// sum that comes out infinite or NaN is therefore taken again on the float matrix unit (float_sums), which keeps the
+// infinities and the top of the range; a 3x3 convolution gives NaN there, as the Winograd transforms do. Weights keep their
+// value at the top of the range (their first plane is cut, not rounded, where it would overflow). Below 2^-110 (7.7e-34)
+// the last planes fall under the smallest bf16, and an operand keeps fewer bits.
 #include "kgx_gemm_epi.h"
 
+#include <cfloat>
 #include <climits>
 #include <cstring>
 #include <vector>
@@ -46,6 +51,39 @@ __device__ __forceinline__ void split3(const floatx4 (&x)[2], u32x4 (&p)[3]) {
       }
     }
   }
+}
+
+// The products of 16 rows with a packed 16-column block on v_mfma_f32_16x16x4_f32: ap this lane's row (lane % 16) of A at
+// inputs 8 (lane / 16), wp its fragments of W, whose planes add up to the float weights. The steps' shares are summed as
+// the wave pairs' are, so that a sum depends on its row and column alone. All lanes of the wave take part.
+__device__ __forceinline__ floatx4 float_sums(const float* ap, const bf16* wp, int steps) {
+  floatx4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+  for (int w = 0; w < 4; w++) {
+    floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int s = w; s < steps; s += 4) {
+      const floatx4 a[2] = {*(const floatx4*)(ap + s * 32), *(const floatx4*)(ap + s * 32 + 4)};
+      bf16x8 b[3];
+#pragma unroll
+      for (int q = 0; q < 3; q++) b[q] = *(const bf16x8*)(wp + ((size_t)s * 3 + q) * PFRAG);
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        const float wt = (float)b[0][e] + ((float)b[1][e] + (float)b[2][e]);
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e >> 2][e & 3], wt, acc, 0, 0, 0);
+      }
+    }
+    sum += acc;
+  }
+  return sum;
+}
+
+__device__ __forceinline__ bool finite(float v) { return __builtin_fabsf(v) <= FLT_MAX; }
+// Whether any of v is infinite or NaN, for one compare a call: adds 0 or NaN to z.
+__device__ __forceinline__ float add_zeros(float z, floatx4 v) {
+#pragma unroll
+  for (int k = 0; k < 4; k++) z = __builtin_fmaf(v[k], 0.f, z);
+  return z;
 }
 
 template <int MB, int NB, int SC>
@@ -395,6 +433,19 @@ __global__ __launch_bounds__(PNT, MB == 2 ? 4 : 2) void gemm_split_kernel(const 
     floatx4 sum = *(const floatx4*)p;
 #pragma unroll
     for (int q = 1; q < 4; q++) sum += *(const floatx4*)(p + q * BM * ELD);
+    if (__any(!(add_zeros(0.f, sum) == 0.f))) {
+      // The wave's four rows and 64 columns: operand row i is row i / 4 of them, and product q takes columns 4 l + q, so
+      // that lane (g4, l) gets column 4 l + q of row g4 as its first output.
+      const float* xp = A + (size_t)min(m0 + wid * 4 + 32 * v + (r16 >> 2), M - 1) * lda + g4 * 8;
+      const bf16* xw = W + (size_t)(nt * NB + (r16 >> 2)) * steps * 3 * PFRAG + (g4 * 16 + (r16 & 3) * 4) * 8;
+#pragma unroll 1
+      for (int q = 0; q < 4; q++) {
+        const float t = float_sums(xp, xw + q * 8, steps)[0];
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+          if (k == q && !finite(sum[k])) sum[k] = t;
+      }
+    }
     if constexpr (!OWN) {
       *(floatx4*)p = sum;
     } else if (m < M && en < N) {
@@ -543,6 +594,24 @@ __global__ __launch_bounds__(PNT, 2) void gemm_split_lds_kernel(const float* __r
 #pragma unroll
       for (int r = 0; r < 4; r++)
         Et[((wm * WB + i) * 16 + 4 * g4 + r) * ELD + (wn * WC + j) * 16 + r16] = tot[i][j][r];
+  float z = 0.f;
+#pragma unroll
+  for (int i = 0; i < WB; i++)
+#pragma unroll
+    for (int j = 0; j < WC; j++) z = add_zeros(z, tot[i][j]);
+  if (__any(!(z == 0.f))) {
+#pragma unroll 1
+    for (int b = 0; b < WB * WC; b++) {
+      const int row = (wm * WB + b / WC) * 16, col = (wn * WC + b % WC) * 16;
+      if (n0 + col >= N) continue;
+      const floatx4 t = float_sums(A + (size_t)min(m0 + row + r16, M - 1) * lda + g4 * 8,
+                                   W + (size_t)((n0 + col) / 16) * steps * 3 * PFRAG + lane * 8, steps);
+      for (int r = 0; r < 4; r++) {
+        float* p = Et + (row + 4 * g4 + r) * ELD + col + r16;
+        if (!finite(*p)) *p = t[r];
+      }
+    }
+  }
   lds_barrier();
   if constexpr (!OWN) {
     gemm_tile_epilogue<float, EPI, BM, BN, PNT>(Et, g, o, m0, n0, M, N, tid);
@@ -559,17 +628,18 @@ __global__ __launch_bounds__(PNT, 2) void gemm_split_lds_kernel(const float* __r
   }
 }
 
-// The three planes of v (round to nearest even; infinities and NaN keep their first plane).
+// The three planes of v (round to nearest even, but cut where that would be infinite: the next planes hold the rest; an
+// infinity is its first plane alone).
 inline void host_split3(float v, uint16_t* p, size_t plane) {
   for (int q = 0; q < 3; q++) {
     uint32_t u;
     std::memcpy(&u, &v, 4);
-    if ((u & 0x7f800000u) != 0x7f800000u) u += 0x7fffu + ((u >> 16) & 1u);
-    u &= 0xffff0000u;
-    p[q * plane] = (uint16_t)(u >> 16);
+    const uint32_t r = u + 0x7fffu + ((u >> 16) & 1u);
+    const uint32_t hb = ((r & 0x7f800000u) == 0x7f800000u ? u : r) & 0xffff0000u;
+    p[q * plane] = (uint16_t)(hb >> 16);
     float h;
-    std::memcpy(&h, &u, 4);
-    v -= h;
+    std::memcpy(&h, &hb, 4);
+    v = (u & 0x7fffffffu) == 0x7f800000u ? 0.f : v - h;
   }
 }
 
