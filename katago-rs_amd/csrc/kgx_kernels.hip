@@ -1135,8 +1135,12 @@ __global__ __launch_bounds__(ATF_NW * 64) void attn_f32_kernel(const float* __re
   const float* mrow = mask + (size_t)n * HW;
   const int key0 = wave * ATF_WT * 16;
 
-  // Rows past the board are clamped to the last point: its values are finite wherever the board's are, a key past
-  // the board gets probability 0, and a query past it is not stored.
+  // Rows past the board are clamped to the last point; a key past it takes no part (its score is kept out of the maximum,
+  // its numerator and its row of V are 0: the score of a real key may be anything down to -inf, and V infinite), and a
+  // query past it is not stored. Only the last tiles hold such keys.
+  auto on = [&](int t, int r) {
+    return ((ATF_NW - 1) * ATF_WT + t + 1) * 16 <= HW || key0 + 16 * t + 4 * g + r < HW;
+  };
   floatx4 qf[QT][KC];
 #pragma unroll
   for (int qt = 0; qt < QT; qt++) {
@@ -1177,17 +1181,15 @@ __global__ __launch_bounds__(ATF_NW * 64) void attn_f32_kernel(const float* __re
         for (int qt = 0; qt < QT; qt++)
           sc[t][qt] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[t & 1][c][j], qf[qt][c][j], sc[t][qt], 0, 0, 0);
 #pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const bool on = key0 + 16 * t + 4 * g + r < HW;
+    for (int r = 0; r < 4; r++)
 #pragma unroll
-      for (int qt = 0; qt < QT; qt++) sc[t][qt][r] = on ? sc[t][qt][r] + (mk[t][r] * 3e4f - 3e4f) : -1e30f;
-    }
+      for (int qt = 0; qt < QT; qt++) sc[t][qt][r] = on(t, r) ? sc[t][qt][r] + (mk[t][r] * 3e4f - 3e4f) : -FLT_MAX;
   }
   // The wave's softmax numerators relative to its own maximum, and their sum (both over the four lane groups).
   float l[QT];
 #pragma unroll
   for (int qt = 0; qt < QT; qt++) {
-    float m = sc[0][qt][0];
+    float m = -FLT_MAX;
 #pragma unroll
     for (int t = 0; t < ATF_WT; t++)
 #pragma unroll
@@ -1199,7 +1201,7 @@ __global__ __launch_bounds__(ATF_NW * 64) void attn_f32_kernel(const float* __re
     for (int t = 0; t < ATF_WT; t++)
 #pragma unroll
       for (int r = 0; r < 4; r++) {
-        const float p = __expf(sc[t][qt][r] - m);
+        const float p = on(t, r) ? __expf(sc[t][qt][r] - m) : 0.f;
         sc[t][qt][r] = p;
         s += p;
       }
@@ -1222,10 +1224,12 @@ __global__ __launch_bounds__(ATF_NW * 64) void attn_f32_kernel(const float* __re
 #pragma unroll
     for (int r = 0; r < 4; r++)
 #pragma unroll
-      for (int dt = 0; dt < VW; dt++)
+      for (int dt = 0; dt < VW; dt++) {
+        const float v = on(t, r) ? vf[t & 1][r][dt] : 0.f;
 #pragma unroll
         for (int qt = 0; qt < QT; qt++)
-          o[dt][qt] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[t & 1][r][dt], sc[t][qt][r], o[dt][qt], 0, 0, 0);
+          o[dt][qt] = __builtin_amdgcn_mfma_f32_16x16x4f32(v, sc[t][qt][r], o[dt][qt], 0, 0, 0);
+      }
   }
   // Element (dt, r) of a lane is dim VW (4g + r) + dt of its query: 4 VW consecutive dims.
 #pragma unroll
