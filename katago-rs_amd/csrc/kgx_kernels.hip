@@ -1112,6 +1112,8 @@ constexpr int ATF_NW = 4, ATF_KT = (HW + 15) / 16, ATF_WT = (ATF_KT + ATF_NW - 1
 // (5 rows of b10c512h8), 45.3 against 41.2 at 80 and 123 against 114 at 256.
 constexpr int ATF_NARROW_HEADS = 20;
 
+__device__ const float kZeroRow[4] __attribute__((aligned(16))) = {0.f, 0.f, 0.f, 0.f};
+
 template <int D, int QT>
 __global__ __launch_bounds__(ATF_NW * 64) void attn_f32_kernel(const float* __restrict__ qkv,
                                                                const float* __restrict__ mask, int nheads_total, int H,
@@ -1135,9 +1137,9 @@ __global__ __launch_bounds__(ATF_NW * 64) void attn_f32_kernel(const float* __re
   const float* mrow = mask + (size_t)n * HW;
   const int key0 = wave * ATF_WT * 16;
 
-  // Rows past the board are clamped to the last point; a key past it takes no part (its score is kept out of the maximum,
-  // its numerator and its row of V are 0: the score of a real key may be anything down to -inf, and V infinite), and a
-  // query past it is not stored. Only the last tiles hold such keys.
+  // Rows past the board are clamped to the last point, and a query past it is not stored. A key past it takes no part:
+  // its score is -inf, and its row of V is read as zeros (the last point's may be infinite). Only the last tiles hold such
+  // keys.
   auto on = [&](int t, int r) {
     return ((ATF_NW - 1) * ATF_WT + t + 1) * 16 <= HW || key0 + 16 * t + 4 * g + r < HW;
   };
@@ -1157,7 +1159,8 @@ __global__ __launch_bounds__(ATF_NW * 64) void attn_f32_kernel(const float* __re
   vrow_t vf[2][4];
   auto load_v = [&](int t, vrow_t (&v)[4]) {
 #pragma unroll
-    for (int r = 0; r < 4; r++) v[r] = *(const vrow_t*)(vp + (size_t)min(key0 + 16 * t + 4 * g + r, HW - 1) * ldq);
+    for (int r = 0; r < 4; r++)
+      v[r] = *(const vrow_t*)(on(t, r) ? vp + (size_t)(key0 + 16 * t + 4 * g + r) * ldq : kZeroRow);
   };
   float mk[ATF_WT][4];
 #pragma unroll
@@ -1183,7 +1186,7 @@ __global__ __launch_bounds__(ATF_NW * 64) void attn_f32_kernel(const float* __re
 #pragma unroll
     for (int r = 0; r < 4; r++)
 #pragma unroll
-      for (int qt = 0; qt < QT; qt++) sc[t][qt][r] = on(t, r) ? sc[t][qt][r] + (mk[t][r] * 3e4f - 3e4f) : -FLT_MAX;
+      for (int qt = 0; qt < QT; qt++) sc[t][qt][r] = on(t, r) ? sc[t][qt][r] + (mk[t][r] * 3e4f - 3e4f) : -INFINITY;
   }
   // The wave's softmax numerators relative to its own maximum, and their sum (both over the four lane groups).
   float l[QT];
@@ -1201,7 +1204,7 @@ __global__ __launch_bounds__(ATF_NW * 64) void attn_f32_kernel(const float* __re
     for (int t = 0; t < ATF_WT; t++)
 #pragma unroll
       for (int r = 0; r < 4; r++) {
-        const float p = on(t, r) ? __expf(sc[t][qt][r] - m) : 0.f;
+        const float p = __expf(sc[t][qt][r] - m);
         sc[t][qt][r] = p;
         s += p;
       }
@@ -1224,12 +1227,10 @@ __global__ __launch_bounds__(ATF_NW * 64) void attn_f32_kernel(const float* __re
 #pragma unroll
     for (int r = 0; r < 4; r++)
 #pragma unroll
-      for (int dt = 0; dt < VW; dt++) {
-        const float v = on(t, r) ? vf[t & 1][r][dt] : 0.f;
+      for (int dt = 0; dt < VW; dt++)
 #pragma unroll
         for (int qt = 0; qt < QT; qt++)
-          o[dt][qt] = __builtin_amdgcn_mfma_f32_16x16x4f32(v, sc[t][qt][r], o[dt][qt], 0, 0, 0);
-      }
+          o[dt][qt] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[t & 1][r][dt], sc[t][qt][r], o[dt][qt], 0, 0, 0);
   }
   // Element (dt, r) of a lane is dim VW (4g + r) + dt of its query: 4 VW consecutive dims.
 #pragma unroll
