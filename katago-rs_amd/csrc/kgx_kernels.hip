@@ -1112,7 +1112,15 @@ constexpr int ATF_NW = 4, ATF_KT = (HW + 15) / 16, ATF_WT = (ATF_KT + ATF_NW - 1
 // (5 rows of b10c512h8), 45.3 against 41.2 at 80 and 123 against 114 at 256.
 constexpr int ATF_NARROW_HEADS = 20;
 
-__device__ const float kZeroRow[4] __attribute__((aligned(16))) = {0.f, 0.f, 0.f, 0.f};
+// The W floats at byte offset off of [base, base + nbytes), 0 past the range (a buffer load: no branch, no 64-bit address).
+template <int W>
+__device__ __forceinline__ auto range_load(const float* base, int nbytes, int off) {
+  typedef float vec_t __attribute__((ext_vector_type(W)));
+  auto rs = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, nbytes, 0x00020000);
+  if constexpr (W == 4) return __builtin_bit_cast(vec_t, __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0));
+  else if constexpr (W == 2) return __builtin_bit_cast(vec_t, __builtin_amdgcn_raw_buffer_load_b64(rs, off, 0, 0));
+  else return __builtin_bit_cast(vec_t, __builtin_amdgcn_raw_buffer_load_b32(rs, off, 0, 0));
+}
 
 template <int D, int QT>
 __global__ __launch_bounds__(ATF_NW * 64) void attn_f32_kernel(const float* __restrict__ qkv,
@@ -1133,13 +1141,13 @@ __global__ __launch_bounds__(ATF_NW * 64) void attn_f32_kernel(const float* __re
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, g = lane >> 4;
   const float* base = qkv + (size_t)n * HW * ldq;
   const float* kp = base + k_off + kvh * D + 4 * g;
-  const float* vp = base + v_off + kvh * D + VW * l16;
+  const int rbytes = ldq * 4, voff = (v_off + kvh * D + VW * l16) * 4;
   const float* mrow = mask + (size_t)n * HW;
   const int key0 = wave * ATF_WT * 16;
 
   // Rows past the board are clamped to the last point, and a query past it is not stored. A key past it takes no part:
-  // its score is -inf, and its row of V is read as zeros (the last point's may be infinite). Only the last tiles hold such
-  // keys.
+  // its score is -inf, and its row of V lies past the range and reads as zeros (the last point's may be infinite). Only the
+  // last tiles hold such keys.
   auto on = [&](int t, int r) {
     return ((ATF_NW - 1) * ATF_WT + t + 1) * 16 <= HW || key0 + 16 * t + 4 * g + r < HW;
   };
@@ -1160,7 +1168,7 @@ __global__ __launch_bounds__(ATF_NW * 64) void attn_f32_kernel(const float* __re
   auto load_v = [&](int t, vrow_t (&v)[4]) {
 #pragma unroll
     for (int r = 0; r < 4; r++)
-      v[r] = *(const vrow_t*)(on(t, r) ? vp + (size_t)(key0 + 16 * t + 4 * g + r) * ldq : kZeroRow);
+      v[r] = range_load<VW>(base, HW * rbytes, (key0 + 16 * t + 4 * g + r) * rbytes + voff);
   };
   float mk[ATF_WT][4];
 #pragma unroll
