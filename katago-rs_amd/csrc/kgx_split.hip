@@ -433,7 +433,7 @@ __global__ __launch_bounds__(PNT, MB == 2 ? 4 : 2) void gemm_split_kernel(const 
     floatx4 sum = *(const floatx4*)p;
 #pragma unroll
     for (int q = 1; q < 4; q++) sum += *(const floatx4*)(p + q * BM * ELD);
-    if (__any(!(add_zeros(0.f, sum) == 0.f))) {
+    if (__builtin_expect(__any(!(add_zeros(0.f, sum) == 0.f)), 0)) {
       // The wave's four rows and 64 columns: operand row i is row i / 4 of them, and product q takes columns 4 l + q, so
       // that lane (g4, l) gets column 4 l + q of row g4 as its first output.
       const float* xp = A + (size_t)min(m0 + wid * 4 + 32 * v + (r16 >> 2), M - 1) * lda + g4 * 8;
@@ -594,12 +594,14 @@ __global__ __launch_bounds__(PNT, 2) void gemm_split_lds_kernel(const float* __r
 #pragma unroll
       for (int r = 0; r < 4; r++)
         Et[((wm * WB + i) * 16 + 4 * g4 + r) * ELD + (wn * WC + j) * 16 + r16] = tot[i][j][r];
-  float z = 0.f;
+  floatx4 z = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int i = 0; i < WB; i++)
 #pragma unroll
-    for (int j = 0; j < WC; j++) z = add_zeros(z, tot[i][j]);
-  if (__any(!(z == 0.f))) {
+    for (int j = 0; j < WC; j++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) z[r] = __builtin_fmaf(tot[i][j][r], 0.f, z[r]);
+  if (__builtin_expect(__any(!(add_zeros(0.f, z) == 0.f)), 0)) {
 #pragma unroll 1
     for (int b = 0; b < WB * WC; b++) {
       const int row = (wm * WB + b / WC) * 16, col = (wn * WC + b % WC) * 16;
