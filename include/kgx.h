@@ -300,6 +300,12 @@ int kg_conv_weight_load(int ks, int ic, int oc, int split, int q, int wave, int 
                         int* dst_row, int* dst_chunk);
 /* The stored chunk of logical 16-byte chunk `chunk` of LDS weight row `row` (what the fragment reads address). */
 int kg_conv_weight_chunk(int row, int chunk);
+/* Float handles' products on the bf16 matrix units: a 3x3 convolution (ks 3) of k -> cols channels over `rows` pixels, or a
+ * GEMM (ks 1) of `rows` rows and `cols` columns over k inputs (k a multiple of 32, cols of 4). The launch's workgroup
+ * count, its tile, and the row and column tile of workgroup `workgroup` (-1 when it exits at once). No counterpart in
+ * the reference: the rule and index map that the kernels use, for host-side checks. */
+int kg_float_tile_of(int ks, int rows, int cols, int k, int workgroup, int* grid, int* tile_rows, int* tile_cols,
+                     int* row_tile, int* col_tile);
 /* The nested-bottleneck junction launch (one block's exit 1x1 convolution, 192 -> 384, and the next block's entry
  * 1x1, 384 -> 192, in one kernel) over `pixels` pixels: its workgroup count, and the 48-pixel tile that workgroup
  * `workgroup` computes (-1 when it exits at once). (Up to 8192 pixels the launch takes 16- or 32-pixel tiles in order

@@ -619,6 +619,20 @@ int kg_conv_weight_load(int ks, int ic, int oc, int split, int q, int wave, int 
   });
 }
 
+int kg_float_tile_of(int ks, int rows, int cols, int k, int workgroup, int* grid, int* tile_rows, int* tile_cols,
+                     int* row_tile, int* col_tile) {
+  return guarded([&] {
+    if (!grid || !tile_rows || !tile_cols || !row_tile || !col_tile) throw std::runtime_error("null output");
+    if ((ks != 1 && ks != 3) || rows < 1 || cols < 1 || k < 1 || (ks == 1 && !kgx::gemm_split_fits(cols, k, 0)))
+      throw std::runtime_error("bad product shape");
+    const kgx::SplitGeometry g = kgx::split_geometry(ks, rows, cols, k, std::max(workgroup, 0), *row_tile, *col_tile);
+    *grid = g.grid;
+    *tile_rows = g.tile_rows;
+    *tile_cols = g.tile_cols;
+    if (workgroup < 0 || workgroup >= g.grid) throw std::runtime_error("workgroup out of range");
+  });
+}
+
 int kg_conv_weight_chunk(int row, int chunk) {
   return row >= 0 && chunk >= 0 && chunk < 8 ? kgx::conv_igemm_weight_chunk(row, chunk) : -1;
 }

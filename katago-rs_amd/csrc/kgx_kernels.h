@@ -201,6 +201,12 @@ void launch_conv_small(int prec, int mb, const void* x, int ldx, const void* w, 
 // conv_split_pack_weights, OC % 4 == 0.
 void conv_split_pack_weights(const float* w, int oc, int ic, std::vector<float>& out);
 void launch_conv_split(const float* x, int ldx, int IC, const void* w, int OC, const ConvOut& o, int B, hipStream_t s);
+// The grid and tile that a float 3x3 convolution (ks 3: M pixels, K -> N channels) or GEMM (ks 1: M x N over K) of kgx_split.hip
+// runs on, and the tiles of workgroup g (-1 when it exits at once).
+struct SplitGeometry {
+  int grid = 0, tile_rows = 0, tile_cols = 0;
+};
+SplitGeometry split_geometry(int ks, int M, int N, int K, int g, int& row_tile, int& col_tile);
 // The value a float becomes as a compute-type operand (round to nearest even), as a float.
 float conv_round_operand(float v, int prec);
 

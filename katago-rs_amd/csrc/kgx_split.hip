@@ -34,6 +34,20 @@ namespace {
 constexpr int PNT = 512, PCH = 64, PSTEPS = 18, PHALO = POS + 1;
 constexpr int PFRAG = 64 * 8;  // elements of a packed weight fragment
 
+// Row tile mt, column tile nt of workgroup g: the column tiles of a row tile on one XCD (workgroup g runs on XCD g mod 8),
+// where they share its L2 for the rows.
+__host__ __device__ inline void split_tile_of(int g, int ntl, int& mt, int& nt) {
+  const int slot = g >> 3, u = slot / ntl;
+  nt = slot - u * ntl;
+  mt = u * 8 + (g & 7);
+}
+inline int split_grid(int M, int bm, int ntl) { return round_up((M + bm - 1) / bm, 8) * ntl; }
+// The workgroups of the XCD that has most of them, the first: a round of the chip is 32 of these (one per CU), whatever the
+// others have. (12 row tiles x 18 column tiles are 216 workgroups, under one round of 256 CUs, but 36 on XCD 0 to 3.)
+inline long split_busiest(int M, int N, int bm, int bn) {
+  return (long)(((M + bm - 1) / bm + 7) / 8) * ((N + bn - 1) / bn);
+}
+
 // x as three bf16 planes, eight values at a time (16 bytes per plane).
 __device__ __forceinline__ void split3(const floatx4 (&x)[2], u32x4 (&p)[3]) {
   typedef float floatx2 __attribute__((ext_vector_type(2)));
@@ -99,8 +113,8 @@ __global__ __launch_bounds__(PNT, 1) void conv3_split_kernel(const float* __rest
   const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wv = wid & 3, wr = WM == 2 ? (wid >> 2) * WB * 16 : 0, wc = WN == 2 ? (wid >> 2) * WC : 0;  // steps, row, block
   const int r16 = lane & 15, g4 = lane >> 4;
-  // The column tiles of a pixel tile on one XCD (workgroup g runs on XCD g mod 8): they share its L2 for the rows.
-  const int slot = blockIdx.x >> 3, u = slot / ntl, nt = slot - u * ntl, mt = u * 8 + (blockIdx.x & 7);
+  int mt, nt;
+  split_tile_of(blockIdx.x, ntl, mt, nt);
   const int m0 = mt * BM, n0 = nt * BN;
   if (m0 >= M) return;
 
@@ -330,7 +344,8 @@ __global__ __launch_bounds__(PNT, MB == 2 ? 4 : 2) void gemm_split_kernel(const 
   const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wv = wid & 3, wr = WM == 2 ? (wid >> 2) * WB * 16 : 0, wc = WN == 2 ? (wid >> 2) * WC : 0;
   const int r16 = lane & 15, g4 = lane >> 4;
-  const int slot = blockIdx.x >> 3, u = slot / ntl, nt = slot - u * ntl, mt = u * 8 + (blockIdx.x & 7);
+  int mt, nt;
+  split_tile_of(blockIdx.x, ntl, mt, nt);
   const int m0 = mt * BM, n0 = nt * BN;
   if (m0 >= M) return;
 
@@ -476,7 +491,8 @@ __global__ __launch_bounds__(PNT, 2) void gemm_split_lds_kernel(const float* __r
   __shared__ __align__(1024) char smem[2 * BUF];
   const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wid >> 2, wn = wid & 3, r16 = lane & 15, g4 = lane >> 4;
-  const int slot = blockIdx.x >> 3, u = slot / ntl, nt = slot - u * ntl, mt = u * 8 + (blockIdx.x & 7);
+  int mt, nt;
+  split_tile_of(blockIdx.x, ntl, mt, nt);
   const int m0 = mt * BM, n0 = nt * BN;
   if (m0 >= M) return;
 
@@ -669,8 +685,7 @@ void conv_split_pack_weights(const float* w, int oc, int ic, std::vector<float>&
 
 template <int MB, int NB>
 static void split_launch(const float* x, int ldx, int IC, const bf16* w, int OC, const ConvOut& o, int M, hipStream_t s) {
-  const int ntl = (OC + 16 * NB - 1) / (16 * NB), nch = (IC + PCH - 1) / PCH;
-  const int grid = round_up((M + 16 * MB - 1) / (16 * MB), 8) * ntl;
+  const int ntl = (OC + 16 * NB - 1) / (16 * NB), nch = (IC + PCH - 1) / PCH, grid = split_grid(M, 16 * MB, ntl);
   auto go = [&](auto kernel) { launch_k(kernel, grid, PNT, 0, s, x, ldx, IC, w, nch, OC, M, ntl, o); };
   const int sfl = store_flags(o);
   switch ((sfl & SF_EMIT) && o.emit.act != ACT_MISH ? -1 : sfl) {  // the store cases of igemm_launch
@@ -682,31 +697,33 @@ static void split_launch(const float* x, int ldx, int IC, const bf16* w, int OC,
   }
 }
 
+// The tile (16 mb pixels x 16 nb channels) whose rounds (of one workgroup per CU: up to 105 KB of LDS) cost least, a round
+// taking time in proportion to the tile's 16 x 16 blocks and a fixed part (staging, epilogue) of about six blocks'
+// (measured at 192 input channels: 11.3, 23.5 and 30 us for 6, 18 and 24 blocks).
+static const int (&conv_split_tile(int M, int OC))[2] {
+  static const int tiles[4][2] = {{6, 4}, {6, 3}, {6, 2}, {3, 2}};
+  int best = 0;
+  long cost = 0;
+  for (int k = 0; k < 4; k++) {
+    const int mb = tiles[k][0], nb = tiles[k][1];
+    const long c = (split_busiest(M, OC, 16 * mb, 16 * nb) + 31) / 32 * (mb * nb + 6);
+    if (k == 0 || c < cost) best = k, cost = c;
+  }
+  return tiles[best];
+}
+
 void launch_conv_split(const float* x, int ldx, int IC, const void* w, int OC, const ConvOut& o, int B, hipStream_t s) {
   if (IC % 8 || ldx % 4 || OC % 4 || (o.y && o.ldy % 4) || (o.yt && o.ldyt % 4) || (o.colbias && o.ld_colbias % 4) ||
       (o.emit.scale && o.emit.ld % 4) || ((uintptr_t)x | (uintptr_t)w) % 16 || o.pool.psum)
     throw std::runtime_error("conv_split: channel counts must be multiples of 8 (inputs) and 4 (outputs)");
   const int M = B * HW;
   if (M <= 0) return;
-  // The tile whose rounds of 256 workgroups (one per CU: up to 105 KB of LDS) cost least, a round taking time in
-  // proportion to the tile's 16 x 16 blocks and a fixed part (staging, epilogue) of about six blocks' (measured at 192
-  // input channels: 11.3, 23.5 and 30 us for 6, 18 and 24 blocks).
-  int best = 0;
-  long cost = 0;
-  const int tiles[4][2] = {{6, 4}, {6, 3}, {6, 2}, {3, 2}};
-  for (int k = 0; k < 4; k++) {
-    const int mb = tiles[k][0], nb = tiles[k][1];
-    const long wgs = (long)((M + 16 * mb - 1) / (16 * mb)) * ((OC + 16 * nb - 1) / (16 * nb));
-    const long c = (wgs + 255) / 256 * (mb * nb + 6);
-    if (k == 0 || c < cost) best = k, cost = c;
-  }
   const bf16* wp = (const bf16*)w;
-  switch (best) {
-    case 0: split_launch<6, 4>(x, ldx, IC, wp, OC, o, M, s); break;
-    case 1: split_launch<6, 3>(x, ldx, IC, wp, OC, o, M, s); break;
-    case 2: split_launch<6, 2>(x, ldx, IC, wp, OC, o, M, s); break;
-    default: split_launch<3, 2>(x, ldx, IC, wp, OC, o, M, s);
-  }
+  const int(&t)[2] = conv_split_tile(M, OC);
+  if (t[0] == 3) split_launch<3, 2>(x, ldx, IC, wp, OC, o, M, s);
+  else if (t[1] == 2) split_launch<6, 2>(x, ldx, IC, wp, OC, o, M, s);
+  else if (t[1] == 3) split_launch<6, 3>(x, ldx, IC, wp, OC, o, M, s);
+  else split_launch<6, 4>(x, ldx, IC, wp, OC, o, M, s);
   KGX_CHECK_LAUNCH();
 }
 
@@ -731,19 +748,37 @@ void gemm_split_pack_weights(const float* w, int N, int K, std::vector<float>& o
 }
 
 // The row tile (32 x 64, 96 x 64 or, with at least four steps, 128 x 128 in LDS) whose rounds take least, by times in
-// us of a round of one workgroup per CU (two of the 32-row tile) fitted to measurements: 96 x 64 over 16 steps 14.0 a
-// round (10 rounds at 3610 rows x 4096 columns), 128 x 128 24.8 (4 rounds of the same) and 19.6 over 12 steps (1083 x
-// 1536), 32 x 64 8 and 17 over 12 and 48 steps in one round of one workgroup per CU, 59 over 16 and 64 steps on
-// average in two rounds of two (3610 x 512).
+// us of a round of one workgroup per CU of the busiest XCD (two of the 32-row tile) fitted to kernel traces: 96 x 64 over 12
+// steps 12.5-12.9 in one round, 21.2 in two, 42.1 in four, over 48 steps 59 in two; 128 x 128 over 12 steps 20.1-20.8 in
+// one and 39.6-41.5 in two, over 48 steps 64 in one, over 16 steps 99 in four; 32 x 64 over 12 and 48 steps 7.5 and 19
+// at one workgroup per CU, over 12 steps 12.2 at two, over 16 and 64 steps 59 on average in two rounds of two. Counted over
+// the whole chip instead (12 x 18 tiles of 96 x 64 are under 256 workgroups, but 36 on four XCDs) the q|k|v projection of 3
+// rows of b10c384h6 ran on 96 rows in 22.0 us, where 128 takes 20.8.
 int gemm_split_rows(int M, int N, int K) {
   const int steps = K / 32;
-  auto wgs = [&](int rows, int cols) { return (long)((M + rows - 1) / rows) * ((N + cols - 1) / cols); };
-  const long w32 = wgs(32, 64), w96 = wgs(96, 64), w128 = wgs(128, 128);
-  const double t32 = w32 <= 256 ? 0.26 * steps + 5 : (w32 + 511) / 512 * (0.65 * steps + 5);
-  const double t96 = (w96 + 255) / 256 * (0.6 * steps + 4), t128 = (w128 + 255) / 256 * (1.2 * steps + 5);
+  const long w32 = split_busiest(M, N, 32, 64), w96 = split_busiest(M, N, 96, 64), w128 = split_busiest(M, N, 128, 128);
+  const double t32 = w32 <= 32 ? 0.26 * steps + 5 : (w32 + 63) / 64 * (0.65 * steps + 5);
+  const double t96 = (w96 + 31) / 32 * (0.55 * steps + 4) + 2, t128 = (w128 + 31) / 32 * (1.22 * steps + 5.5);
   // (Its weights' offsets are 32-bit.)
   if (steps >= 4 && t128 < t96 && t128 < t32 && 6.0 * (N + 64) * K < INT_MAX) return 128;
   return t96 <= t32 ? 96 : 32;
+}
+
+SplitGeometry split_geometry(int ks, int M, int N, int K, int g, int& row_tile, int& col_tile) {
+  SplitGeometry r;
+  if (ks == 3) {
+    const int(&t)[2] = conv_split_tile(M, N);
+    r.tile_rows = 16 * t[0];
+    r.tile_cols = 16 * t[1];
+  } else {
+    r.tile_rows = gemm_split_rows(M, N, K);
+    r.tile_cols = r.tile_rows == 128 ? 128 : 64;
+  }
+  const int ntl = (N + r.tile_cols - 1) / r.tile_cols;
+  r.grid = split_grid(M, r.tile_rows, ntl);
+  split_tile_of(g, ntl, row_tile, col_tile);
+  if ((long)row_tile * r.tile_rows >= M) row_tile = col_tile = -1;
+  return r;
 }
 
 template <int MB, int EPI>
@@ -755,7 +790,7 @@ static auto gemm_split_pick() {
 template <int MB>
 static void gemm_split_launch(const GemmArgs& g, int epi, hipStream_t s) {
   constexpr int BN = MB == 8 ? 128 : 64;
-  const int ntl = (g.N + BN - 1) / BN, grid = round_up((g.M + 16 * MB - 1) / (16 * MB), 8) * ntl;
+  const int ntl = (g.N + BN - 1) / BN, grid = split_grid(g.M, 16 * MB, ntl);
   auto go = [&](auto kernel) {
     launch_k(kernel, grid, PNT, 0, s, (const float*)g.A, (const bf16*)g.Bt, (int)g.lda, g.M, g.N, g.K, ntl, g);
   };

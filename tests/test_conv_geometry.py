@@ -161,3 +161,34 @@ def test_rmsnorm_rows_cover_each_row_once_from_its_tile_xcd(kgx, channels, regio
             if count and region in (64, 96, 128, 192):
                 assert (first // region) % 8 == g % 8 and (first + count - 1) // region == first // region, (g, first)
         assert set(seen) == set(range(rows)) and all(v == 1 for v in seen.values()), (channels, region, batch)
+
+
+# (ks, rows, cols, k) of float products: a board to 192 of the convolutions, a row to 48 of the token GEMMs' shapes.
+FLOAT_SHAPES = [(3, b * 361, oc, ic) for b in (1, 11, 22, 45, 192) for ic, oc in ((192, 192), (128, 160), (64, 72))] + \
+               [(1, b * 361, n, k) for b in (1, 3, 10, 48) for n, k in ((1152, 384), (384, 1536), (192, 384), (100, 96))]
+
+
+@pytest.mark.parametrize("ks,rows,cols,k", FLOAT_SHAPES)
+def test_float_tiles_are_computed_once_on_one_xcd_per_row_tile(kgx, ks, rows, cols, k):
+    grid, tr, tc = kgx.float_tile_of(ks, rows, cols, k, 0)[:3]
+    seen = collections.Counter()
+    for wg in range(grid):
+        mt, nt = kgx.float_tile_of(ks, rows, cols, k, wg)[3:]
+        if mt < 0:
+            continue
+        assert wg % 8 == mt % 8
+        seen[(mt, nt)] += 1
+    assert set(seen) == {(m, n) for m in range(-(-rows // tr)) for n in range(-(-cols // tc))}
+    assert all(v == 1 for v in seen.values())
+    with pytest.raises(kgx.KgError, match="workgroup out of range"):
+        kgx.float_tile_of(ks, rows, cols, k, grid)
+
+
+# Products whose busiest XCD the rule's tile leaves at one workgroup per CU (32), where another tile has fewer workgroups
+# than there are CUs and yet more than 32 on some XCD: three rows of b10c384h6's q|k|v projection (12 row tiles x 18
+# column tiles of 96 x 64), and 11 boards of 192 -> 192 (42 x 6 tiles of 96 x 32).
+@pytest.mark.parametrize("ks,rows,cols,k", [(1, 3 * 361, 1152, 384), (3, 11 * 361, 192, 192)])
+def test_float_tile_rule_counts_the_busiest_xcd(kgx, ks, rows, cols, k):
+    grid = kgx.float_tile_of(ks, rows, cols, k, 0)[0]
+    load = collections.Counter(wg % 8 for wg in range(grid) if kgx.float_tile_of(ks, rows, cols, k, wg)[3] >= 0)
+    assert max(load.values()) <= 32, load
