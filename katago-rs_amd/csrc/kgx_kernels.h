@@ -135,15 +135,16 @@ struct GemmArgs {
   // Activation of the compute-type output alone (ACT_ID or ACT_MISH): out.yt = act(C), as the mish FFN's h.
   int yt_act = ACT_ID;
   QkvEpi qkv;
-  bool split3 = false;   // float GEMM whose Bt is the upload of gemm_split_pack_weights (kgx_split.hip)
+  bool split3 = false;   // float GEMM whose Bt was made by launch_gemm_split_pack (kgx_split.hip)
   bool vec_epi = false;  // set by launch_gemm: the four-column vector epilogue applies
 };
 void launch_gemm(int prec, const GemmArgs& g, hipStream_t s);
 // Float GEMMs on bf16 matrix cores (kgx_split.hip): whether N columns over K (a q|k|v projection of head dim dq, or 0)
-// fit, the packed weights w [N][K], the rows of the row tile over M rows (row tile r on XCD r mod 8), and the launch
-// with launch_gemm's epilogue `epi`.
+// fit, the bytes of the packed weights and their packing from device floats w [N][K], the rows of the row tile over M rows
+// (row tile r on XCD r mod 8), and the launch with launch_gemm's epilogue `epi`.
 bool gemm_split_fits(int N, int K, int dq);
-void gemm_split_pack_weights(const float* w, int N, int K, std::vector<float>& out);
+size_t gemm_split_bytes(int N, int K);
+void launch_gemm_split_pack(const float* w, int N, int K, void* out, hipStream_t s);
 int gemm_split_rows(int M, int N, int K);
 void launch_gemm_split(const GemmArgs& g, int epi, hipStream_t s);
 // The rows of the row tile that launch_gemm runs a plain GEMM of these sizes on (row tile r on XCD r mod 8).
@@ -197,9 +198,10 @@ void launch_conv_igemm(int prec, int ks, const void* x, int ldx, int IC, const v
 int conv_small_mb(int ks, int ic, int icp, int oc, int M);
 void launch_conv_small(int prec, int mb, const void* x, int ldx, const void* w, int icp, int OC, const ConvOut& o, int M,
                        int pbn, hipStream_t s);
-// Float 3x3 convolution on bf16 matrix cores (kgx_split.hip): x float NHWC rows of ldx (IC % 8 == 0), w the upload of
-// conv_split_pack_weights, OC % 4 == 0.
-void conv_split_pack_weights(const float* w, int oc, int ic, std::vector<float>& out);
+// Float 3x3 convolution on bf16 matrix cores (kgx_split.hip): x float NHWC rows of ldx (IC % 8 == 0), OC % 4 == 0, w the
+// conv_split_bytes that launch_conv_split_pack makes of device floats [oc][ic][3][3].
+size_t conv_split_bytes(int oc, int ic);
+void launch_conv_split_pack(const float* w, int oc, int ic, void* out, hipStream_t s);
 void launch_conv_split(const float* x, int ldx, int IC, const void* w, int OC, const ConvOut& o, int B, hipStream_t s);
 // The grid and tile that a float 3x3 convolution (ks 3: M pixels, K -> N channels) or GEMM (ks 1: M x N over K) of kgx_split.hip
 // runs on, and the tiles of workgroup g (-1 when it exits at once).

@@ -112,6 +112,9 @@ class Net {
   const void* upload_t(const std::vector<float>& v);  // converted to the compute type
   bool gemm_split(int N, int K, int dq) const;
   const void* upload_gemm(const std::vector<float>& w, int N, int K, int dq);
+  // The `bytes` that `pack` (device floats, output) makes of w, which holds `count` floats, on the device.
+  const void* upload_packed(const std::vector<float>& w, size_t count, size_t bytes,
+                            const std::function<void(const float*, void*)>& pack);
   size_t tsize() const { return prec_ == PREC_F32 ? 4 : 2; }
 
   // Planning.
@@ -182,6 +185,7 @@ class Net {
   int wino_tm_ = 4;
   int nin_ = 0, nglob_ = 0, nmeta_ = 0, row_len_ = 0;
   std::vector<std::unique_ptr<DeviceBuffer>> mem_;
+  std::unique_ptr<DeviceBuffer> stage_;  // floats being packed, while the network is built
   std::vector<Op> ops_;
 
   // Inputs / outputs and per-row board data.

@@ -138,9 +138,26 @@ bool Net::gemm_split(int N, int K, int dq) const { return conv_mode_ == CONV_SPL
 
 const void* Net::upload_gemm(const std::vector<float>& w, int N, int K, int dq) {
   if (!gemm_split(N, K, dq)) return upload_t(w);
-  std::vector<float> p;
-  gemm_split_pack_weights(w.data(), N, K, p);
-  return upload_f(p);
+  return upload_packed(w, (size_t)N * K, gemm_split_bytes(N, K),
+                       [=](const float* d, void* out) { launch_gemm_split_pack(d, N, K, out, nullptr); });
+}
+
+const void* Net::upload_packed(const std::vector<float>& w, size_t count, size_t bytes,
+                               const std::function<void(const float*, void*)>& pack) {
+  if (w.size() != count) throw std::runtime_error("internal: weight count");
+  if (primary_) return take_upload(bytes);
+  const size_t need = w.size() * sizeof(float);
+  if (!stage_ || stage_->bytes < need) {
+    stage_ = std::make_unique<DeviceBuffer>();
+    KGX_HIP(hipMalloc(&stage_->ptr, need));
+    stage_->bytes = need;
+  }
+  void* d = alloc_bytes(bytes);
+  // (The copy, the packing and the next copy are ordered on the null stream; build() waits for the last.)
+  KGX_HIP(hipMemcpy(stage_->ptr, w.data(), need, hipMemcpyHostToDevice));
+  pack((const float*)stage_->ptr, d);
+  uploads_.emplace_back(d, bytes);
+  return d;
 }
 
 RowProg Net::row_prog_base() const {
@@ -371,9 +388,9 @@ std::shared_ptr<ConvOut> Net::emit_conv(const ConvDesc& c, const void* x, int ld
   // must not depend on it.
   if (k3 && conv_mode_ == CONV_SPLIT && (long)c.ic * c.oc <= 256 * 256 && !nchw && c.ic % 8 == 0 && ldx % 4 == 0 && c.oc % 4 == 0 &&
       (!o.y || o.ldy % 4 == 0) && (!o.yt || o.ldyt % 4 == 0) && (!o.colbias || o.ld_colbias % 4 == 0) && !o.pool.psum) {
-    std::vector<float> w;
-    conv_split_pack_weights(c.w.data(), c.oc, c.ic, w);
-    const float* dW = upload_f(w);
+    const void* dW = upload_packed(c.w, (size_t)oc * ic * 9, conv_split_bytes(oc, ic), [=](const float* d, void* to) {
+      launch_conv_split_pack(d, oc, ic, to, nullptr);
+    });
     const float* xf = (const float*)x;
     Op op;
     op.launch = [=](hipStream_t s, int B) { launch_conv_split(xf, ldx, ic, dW, oc, *out, B, s); };
@@ -1201,6 +1218,7 @@ void Net::build(const ModelDesc& m) {
     }
   }
   if (!primary_) KGX_HIP(hipDeviceSynchronize());
+  stage_.reset();
 }
 
 void Net::run_ops(int B, hipStream_t s) {

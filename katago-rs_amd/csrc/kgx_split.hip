@@ -24,8 +24,6 @@
 
 #include <cfloat>
 #include <climits>
-#include <cstring>
-#include <vector>
 
 namespace kgx {
 
@@ -646,41 +644,68 @@ __global__ __launch_bounds__(PNT, 2) void gemm_split_lds_kernel(const float* __r
   }
 }
 
-// The three planes of v (round to nearest even, but cut where that would be infinite: the next planes hold the rest; an
-// infinity is its first plane alone).
-inline void host_split3(float v, uint16_t* p, size_t plane) {
+// The three planes of a weight (round to nearest even, but cut where that would be infinite: the next planes hold the rest;
+// an infinity is its first plane alone).
+__device__ __forceinline__ void split_weight(float v, unsigned short (&p)[3]) {
+#pragma unroll
   for (int q = 0; q < 3; q++) {
-    uint32_t u;
-    std::memcpy(&u, &v, 4);
-    const uint32_t r = u + 0x7fffu + ((u >> 16) & 1u);
-    const uint32_t hb = ((r & 0x7f800000u) == 0x7f800000u ? u : r) & 0xffff0000u;
-    p[q * plane] = (uint16_t)(hb >> 16);
-    float h;
-    std::memcpy(&h, &hb, 4);
-    v = (u & 0x7fffffffu) == 0x7f800000u ? 0.f : v - h;
+    const unsigned u = __builtin_bit_cast(unsigned, v), r = u + 0x7fffu + ((u >> 16) & 1u);
+    const unsigned h = ((r & 0x7f800000u) == 0x7f800000u ? u : r) & 0xffff0000u;
+    p[q] = (unsigned short)(h >> 16);
+    v = (u & 0x7fffffffu) == 0x7f800000u ? 0.f : v - __builtin_bit_cast(float, h);
+  }
+}
+
+// Packs the weights as the kernels read them, eight elements of the three planes per thread, `frags` fragment triples (64
+// threads each). GEMM (CONV false): w [N][K] -> [16-column block][step][plane], lane l, element e holding column l % 16,
+// input 32 step + 8 (l / 16) + e. Convolution: w [N][K][3][3] -> [16-column block][chunk][step][plane], input channel 64
+// chunk + 32 (step % 2) + 8 (l / 16) + e at tap step / 2. Zeros past N and K. On the device: a handle of b10c384h6 took 41 ms to
+// create with this on the host, 26 ms with it here; one of b18c384nbt 112 and 19 ms.
+template <bool CONV>
+__global__ __launch_bounds__(256) void split_pack_kernel(const float* __restrict__ w, int N, int K, int steps, long frags,
+                                                         u32x4* __restrict__ out) {
+  const long f = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (f >= frags) return;
+  const int lane = threadIdx.x & 63;
+  const long cb = f / steps;
+  const int s = (int)(f - cb * steps), st = CONV ? s % PSTEPS : 0;  // convolution: step s is chunk s / 18, step s % 18
+  const long col = cb * 16 + (lane & 15);
+  const int k0 = (CONV ? s / PSTEPS * PCH + (st & 1) * 32 : s * 32) + (lane >> 4) * 8;
+  unsigned short p[8][3];
+#pragma unroll
+  for (int e = 0; e < 8; e++) {
+    const bool on = col < N && k0 + e < K;
+    split_weight(on ? w[CONV ? ((size_t)col * K + k0 + e) * 9 + st / 2 : (size_t)col * K + k0 + e] : 0.f, p[e]);
+  }
+#pragma unroll
+  for (int q = 0; q < 3; q++) {
+    u32x4 v;
+#pragma unroll
+    for (int k = 0; k < 4; k++) v[k] = p[2 * k][q] | (unsigned)p[2 * k + 1][q] << 16;
+    out[(f * 3 + q) * 64 + lane] = v;
   }
 }
 
 }  // namespace
 
-// w [oc][ic][3][3] -> fragments [16-column block][chunk][step][plane], lane l, element e holding column l % 16, input
-// channel 64 chunk + 32 (step % 2) + 8 (l / 16) + e at tap step / 2; two bf16 per float of `out`, zeros past oc and ic
-// (up to a multiple of 192 columns, so that every tile width reads whole packed blocks).
-void conv_split_pack_weights(const float* w, int oc, int ic, std::vector<float>& out) {
-  const int cbs = round_up(oc, 192) / 16, nch = (ic + PCH - 1) / PCH;
-  std::vector<uint16_t> p((size_t)cbs * nch * PSTEPS * 3 * PFRAG, 0);
-  for (int cb = 0; cb < cbs; cb++)
-    for (int kc = 0; kc < nch; kc++)
-      for (int s = 0; s < PSTEPS; s++)
-        for (int l = 0; l < 64; l++)
-          for (int e = 0; e < 8; e++) {
-            const int col = cb * 16 + l % 16, i = kc * PCH + (s & 1) * 32 + (l / 16) * 8 + e;
-            if (col >= oc || i >= ic) continue;
-            host_split3(w[((size_t)col * ic + i) * 9 + s / 2],
-                        p.data() + (((size_t)cb * nch + kc) * PSTEPS + s) * 3 * PFRAG + l * 8 + e, PFRAG);
-          }
-  out.resize(p.size() / 2);
-  std::memcpy(out.data(), p.data(), p.size() * 2);
+// Convolution weights are packed up to a multiple of 192 columns, so that every tile width reads whole blocks.
+static long conv_split_steps(int ic) { return (long)((ic + PCH - 1) / PCH) * PSTEPS; }
+static long conv_split_frags(int oc, int ic) { return round_up(oc, 192) / 16 * conv_split_steps(ic); }
+static long gemm_split_frags(int N, int K) { return (long)round_up(N, 64) / 16 * (K / 32); }
+
+size_t conv_split_bytes(int oc, int ic) { return conv_split_frags(oc, ic) * 3 * PFRAG * sizeof(bf16); }
+size_t gemm_split_bytes(int N, int K) { return gemm_split_frags(N, K) * 3 * PFRAG * sizeof(bf16); }
+
+void launch_conv_split_pack(const float* w, int oc, int ic, void* out, hipStream_t s) {
+  const long n = conv_split_frags(oc, ic);
+  launch_k(split_pack_kernel<true>, (unsigned)((n + 3) / 4), 256, 0, s, w, oc, ic, (int)conv_split_steps(ic), n, (u32x4*)out);
+  KGX_CHECK_LAUNCH();
+}
+
+void launch_gemm_split_pack(const float* w, int N, int K, void* out, hipStream_t s) {
+  const long n = gemm_split_frags(N, K);
+  launch_k(split_pack_kernel<false>, (unsigned)((n + 3) / 4), 256, 0, s, w, N, K, K / 32, n, (u32x4*)out);
+  KGX_CHECK_LAUNCH();
 }
 
 template <int MB, int NB>
@@ -728,24 +753,6 @@ void launch_conv_split(const float* x, int ldx, int IC, const void* w, int OC, c
 }
 
 bool gemm_split_fits(int N, int K, int dq) { return K % 32 == 0 && N % 4 == 0 && (dq == 0 || 64 % dq == 0); }
-
-// w [N][K] -> fragments [16-column block][step][plane], lane l, element e holding column l % 16, input 32 step +
-// 8 (l / 16) + e; two bf16 per float of `out`, zeros past N up to a multiple of 64 columns.
-void gemm_split_pack_weights(const float* w, int N, int K, std::vector<float>& out) {
-  const int cbs = round_up(N, 64) / 16, steps = K / 32;
-  std::vector<uint16_t> p((size_t)cbs * steps * 3 * PFRAG, 0);
-  for (int cb = 0; cb < cbs; cb++)
-    for (int s = 0; s < steps; s++)
-      for (int l = 0; l < 64; l++)
-        for (int e = 0; e < 8; e++) {
-          const int col = cb * 16 + l % 16;
-          if (col >= N) continue;
-          host_split3(w[(size_t)col * K + s * 32 + (l / 16) * 8 + e],
-                      p.data() + ((size_t)cb * steps + s) * 3 * PFRAG + l * 8 + e, PFRAG);
-        }
-  out.resize(p.size() / 2);
-  std::memcpy(out.data(), p.data(), p.size() * 2);
-}
 
 // The row tile (32 x 64, 96 x 64 or, with at least four steps, 128 x 128 in LDS) whose rounds take least, by times in
 // us of a round of one workgroup per CU of the busiest XCD (two of the 32-row tile) fitted to kernel traces: 96 x 64 over 12
