@@ -356,20 +356,18 @@ def _outputs(n, want_ownership):
 
 _OUTPUT_FIELDS = ["white_win_prob", "white_loss_prob", "white_no_result_prob", "white_score_mean", "white_score_mean_sq",
                   "white_lead", "var_time_left", "shortterm_winloss_error", "shortterm_score_error"]
+_OUTPUT_KEYS = ["policy", *_OUTPUT_FIELDS, "ownership"]
 
 
 def _output_dicts(outs, owners):
-    """The output structures as one dict of NNOutput fields per row."""
+    """The output structures as one dict of NNOutput fields per row. A row's arrays are copies of its own, so that a
+    caller that keeps one row keeps that row alive and not the batch's."""
     if not len(outs):
         return []
     rec = _records(outs)
-    result = []
-    for i, (policy, *fields) in enumerate(zip(rec["policy_probs"], *(rec[f].tolist() for f in _OUTPUT_FIELDS))):
-        d = {"policy": policy.copy()}
-        d.update(zip(_OUTPUT_FIELDS, fields))
-        d["ownership"] = None if owners is None else owners[i]
-        result.append(d)
-    return result
+    owned = [None] * len(outs) if owners is None else [o.copy() for o in owners]
+    columns = [[p.copy() for p in rec["policy_probs"]], *(rec[f].tolist() for f in _OUTPUT_FIELDS), owned]
+    return [dict(zip(_OUTPUT_KEYS, row)) for row in zip(*columns)]
 
 
 def copy_outputs(raw, P: int, S: int, model_version: int, symmetry, policy_optimism, want_ownership=True):

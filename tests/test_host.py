@@ -245,6 +245,21 @@ def test_copy_outputs_sentinels_follow_every_reference_branch(kgx):
         kgx.copy_outputs(spec.sentinel_row(1, 6)[None], 1, 6, 9, 8, 0.0)
 
 
+def test_output_rows_own_their_memory(kgx):
+    """The policy and ownership of a row belong to it: keeping one row (a cache of evaluations) keeps no other's, and
+    writing to it changes no other's."""
+    import outputs_spec as spec
+    raw = np.stack([spec.sentinel_row(2, 6)] * 3)
+    rows = kgx.copy_outputs(raw, 2, 6, 14, 0, 0.0)
+    for r in rows:
+        for k in ("policy", "ownership"):
+            assert r[k].base is None and r[k].flags.owndata and r[k].flags.writeable, k
+    want = rows[1]["ownership"].copy()
+    rows[0]["ownership"][:] = 7.0
+    assert np.array_equal(rows[1]["ownership"], want)
+    assert all(r["ownership"] is None for r in kgx.copy_outputs(raw, 2, 6, 14, 0, 0.0, want_ownership=False))
+
+
 def test_model_version_table_matches_reference_fixture(kgx):
     """NNModelVersion's per-version input layout against KataGo's own outputs
     (fixtures/upstream-v1.18.2/unit/oracle/modelversion_desc.txt, extracted by tests/golden/gen_modelversion.py):
