@@ -472,8 +472,8 @@ static GemmTile gemm_tile_choice(const GemmArgs& g, int tsize, bool af) {
   return GT_SMALL;
 }
 
-int gemm_row_tile(int prec, int M, int N, int K) {
-  if (prec == PREC_F32 && gemm_split_fits(N, K, 0)) return gemm_split_rows(M, N, K);
+int gemm_row_tile(int prec, int M, int N, int K, bool split3) {
+  if (split3) return gemm_split_rows(M, N, K);
   GemmArgs g;
   g.M = M; g.N = N; g.K = K;
   switch (gemm_tile_choice(g, prec == PREC_F32 ? 4 : 2, false)) {

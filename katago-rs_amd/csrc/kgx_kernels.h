@@ -147,8 +147,9 @@ size_t gemm_split_bytes(int N, int K);
 void launch_gemm_split_pack(const float* w, int N, int K, void* out, hipStream_t s);
 int gemm_split_rows(int M, int N, int K);
 void launch_gemm_split(const GemmArgs& g, int epi, hipStream_t s);
-// The rows of the row tile that launch_gemm runs a plain GEMM of these sizes on (row tile r on XCD r mod 8).
-int gemm_row_tile(int prec, int M, int N, int K);
+// The rows of the row tile that launch_gemm runs a plain GEMM of these sizes on (row tile r on XCD r mod 8); split3: its weights
+// are three-plane ones (GemmArgs).
+int gemm_row_tile(int prec, int M, int N, int K, bool split3);
 
 // Implicit-GEMM 1x1 / 3x3 "same" convolution on 16-bit operands: x compute-type NHWC rows of ldx (IC channels,
 // IC % 8 == 0), w the compute-type conversion of conv_igemm_pack_weights' layout (icp = conv_igemm_icp(ks, IC)),

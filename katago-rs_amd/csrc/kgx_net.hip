@@ -589,8 +589,9 @@ void Net::emit_attention(const BlockDesc& b, int depth) {
   const float* mask = mask_;
   Op rn;
   const int rn_n = res_n_, rn_k = res_k_;
+  const bool rn_split3 = rn_n && gemm_split(rn_n, rn_k, 0);
   rn.launch = [=](hipStream_t s, int B) {
-    const int region = rn_n ? gemm_row_tile(prec, B * HW, rn_n, rn_k) : 0;
+    const int region = rn_n ? gemm_row_tile(prec, B * HW, rn_n, rn_k, rn_split3) : 0;
     launch_rmsnorm_tok(prec, x, c, c, lnw, eps, mask, nrm, c, B * HW, s, region);
   };
   rn.cls = "rmsnorm";
@@ -659,8 +660,9 @@ void Net::emit_ffn(const BlockDesc& b, int depth) {
   const float* mask = mask_;
   Op rn;
   const int rn_n = res_n_, rn_k = res_k_;
+  const bool rn_split3 = rn_n && gemm_split(rn_n, rn_k, 0);
   rn.launch = [=](hipStream_t s, int B) {
-    const int region = rn_n ? gemm_row_tile(prec, B * HW, rn_n, rn_k) : 0;
+    const int region = rn_n ? gemm_row_tile(prec, B * HW, rn_n, rn_k, rn_split3) : 0;
     launch_rmsnorm_tok(prec, x, c, c, lnw, eps, mask, nrm, c, B * HW, s, region);
   };
   rn.cls = "rmsnorm";
