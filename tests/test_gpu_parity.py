@@ -91,11 +91,13 @@ def test_tiny_nets_match_oracle(kgx, synth, oracle, golden, name, prec):
     h.close()
 
 
-@pytest.mark.parametrize("conv,prec", [("wino2", "f32"), ("wino2", "f16"), ("wino2", "bf16"), ("wino4", "f16")])
+@pytest.mark.parametrize("conv,prec", [("wino2", "f32"), ("wino4", "f32"), ("wino2", "f16"), ("wino2", "bf16"),
+                                       ("wino4", "f16")])
 @pytest.mark.parametrize("name", ["t_res", "t_nbt", "t_v8"])
 def test_winograd_variants_match_oracle(kgx, synth, oracle, golden, monkeypatch, name, conv, prec):
-    """The Winograd kernels on every precision (16-bit handles default to the implicit GEMM, float ones to
-    F(4x4,3x3)); the algorithm is chosen when the handle builds its network."""
+    """The Winograd kernels on every precision (16-bit handles default to the implicit GEMM, float ones to the direct sum of
+    three-plane splits up to 256 x 256 channels and to F(4x4,3x3) beyond); the algorithm is chosen when the handle builds
+    its network."""
     monkeypatch.setenv("KGX_CONV", conv)
     g, _ = golden
     mb = synth.write_model(synth.tiny_nets()[name], 1)
@@ -110,6 +112,23 @@ def test_winograd_variants_match_oracle(kgx, synth, oracle, golden, monkeypatch,
     else:
         # Winograd transforms round their transformed operands, not the activations: only the float64 bound.
         check(out, g[f"{name}.out"], net.P, net.S, prec, f"{name} {conv}")
+    h.close()
+
+
+def test_float_matrix_unit_transformer_matches_oracle(kgx, synth, oracle, monkeypatch):
+    """Float handles under KGX_CONV=wino4 run their token GEMMs on the float matrix unit: q|k|v with rotation, the gated
+    output and the residual adds, on its small tiles (3 rows) and its wide ones (90)."""
+    monkeypatch.setenv("KGX_CONV", "wino4")
+    mb = synth.write_model(synth.tiny_nets()["t_tf64"], 2)
+    net = kgx.Net(mb)
+    sp, gl, _ = synth.make_inputs(90, 19, board_sizes=[19, 13, 9])
+    ref = oracle.Model(mb).forward(sp[:3], gl[:3])
+    h = kgx.Handle(net, 90, "f32")
+    for n in (3, 90):
+        print(f"float matrix unit: {n} rows", flush=True)
+        out = h.forward(sp[:n], gl[:n])
+        assert np.isfinite(out).all()
+        check(out[:3], ref, net.P, net.S, "f32", f"t_tf64 wino4, {n} rows")
     h.close()
 
 
