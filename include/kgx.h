@@ -276,8 +276,7 @@ int kg_featurize_rows(int device, int n, const kg_position* rows, int nn_x_len, 
  * kernels.rs); these call the same functions as the kernel and its launcher, and launch nothing.
  * kg_conv_geometry: the configuration that a ks x ks convolution of ic -> oc channels (split: split operands, 1x1
  * only) over `pixels` pixels (batch x 361) runs on the large tiles. (A 3x3 of whole 64-channel stages, up to 192 inputs and
- * outputs, over few pixels, as one board to eleven at 192 outputs, runs conv_small_kernel instead, whose workgroup g
- * takes pixel tile g / column tiles and column tile g mod column tiles of 64, 128 or 192 pixels x 16 channels.) */
+ * outputs, over few pixels, as one board to eleven at 192 outputs, runs on kg_small_tile_of's instead.) */
 typedef struct {
   int grid;                /* workgroups launched */
   int threads;             /* threads per workgroup */
@@ -300,6 +299,14 @@ int kg_conv_weight_load(int ks, int ic, int oc, int split, int q, int wave, int 
                         int* dst_row, int* dst_chunk);
 /* The stored chunk of logical 16-byte chunk `chunk` of LDS weight row `row` (what the fragment reads address). */
 int kg_conv_weight_chunk(int row, int chunk);
+/* The launches that few pixels take on 16-bit handles: a 3x3 convolution of ic -> oc channels, or the junction (ic and oc
+ * unused; its column tile is the entry's 192 channels): the workgroup count (0: the large tiles run, kg_conv_geometry and
+ * kg_junction_tile_of), the tile, and the tiles of workgroup `workgroup`. No counterpart in the reference: the rules
+ * and index maps that the launchers and kernels use, for host-side checks. */
+#define KG_SMALL_CONV3X3 0
+#define KG_SMALL_JUNCTION 1
+int kg_small_tile_of(int kernel, int ic, int oc, int pixels, int workgroup, int* grid, int* tile_rows, int* tile_cols,
+                     int* pixel_tile, int* col_tile);
 /* Float handles' products on the bf16 matrix units: a 3x3 convolution (ks 3) of k -> cols channels over `rows` pixels, or a
  * GEMM (ks 1) of `rows` rows and `cols` columns over k inputs (k a multiple of 32, cols of 4). The launch's workgroup
  * count, its tile, and the row and column tile of workgroup `workgroup` (-1 when it exits at once). No counterpart in
@@ -308,8 +315,8 @@ int kg_float_tile_of(int ks, int rows, int cols, int k, int workgroup, int* grid
                      int* row_tile, int* col_tile);
 /* The nested-bottleneck junction launch (one block's exit 1x1 convolution, 192 -> 384, and the next block's entry
  * 1x1, 384 -> 192, in one kernel) over `pixels` pixels: its workgroup count, and the 48-pixel tile that workgroup
- * `workgroup` computes (-1 when it exits at once). (Up to 8192 pixels the launch takes 16- or 32-pixel tiles in order
- * instead, workgroup g tile g.) No counterpart in the reference: the index map its kernel uses,
+ * `workgroup` computes (-1 when it exits at once). (Up to 8192 pixels the launch runs on kg_small_tile_of's tiles instead.)
+ * No counterpart in the reference: the index map its kernel uses,
  * for host-side checks. */
 int kg_junction_tile_of(int pixels, int workgroup, int* grid, int* tile);
 /* The gpool blocks' tile launch (a global-pooling block's mid activation per 192-pixel tile: pooled features,

@@ -37,7 +37,8 @@ EXPORTS = [
     "kg_get_output", "kg_profile_enable", "kg_profile_reset", "kg_profile_read",
     "kg_model_version_features", "kg_meta_encoder_channels", "kg_copy_outputs", "kg_run_static",
     "kg_get_output_async", "kg_wait", "kg_get_output_eval", "kg_post_outputs",
-    "kg_conv_geometry", "kg_conv_tile_of", "kg_conv_weight_load", "kg_conv_weight_chunk", "kg_float_tile_of", "kg_junction_tile_of", "kg_gpool_tile_of", "kg_l2_touch_line", "kg_rmsnorm_rows_of",
+    "kg_conv_geometry", "kg_conv_tile_of", "kg_conv_weight_load", "kg_conv_weight_chunk", "kg_float_tile_of", "kg_small_tile_of",
+    "kg_junction_tile_of", "kg_gpool_tile_of", "kg_l2_touch_line", "kg_rmsnorm_rows_of",
     "kg_featurize", "kg_featurize_rows", "kg_evaluate_positions",
 ]
 # Completion callback of kg_get_output_async: (user, status).
@@ -214,6 +215,7 @@ def lib():
         L.kg_conv_tile_of.argtypes = [ci, ci, ci, ci, ci, ci, ctypes.POINTER(ci), ctypes.POINTER(ci)]
         L.kg_conv_weight_load.argtypes = [ci, ci, ci, ci, ci, ci, ci] + [ctypes.POINTER(ci)] * 4
         L.kg_conv_weight_chunk.argtypes = [ci, ci]
+        L.kg_small_tile_of.argtypes = [ci] * 5 + [ctypes.POINTER(ci)] * 5
         L.kg_float_tile_of.argtypes = [ci] * 5 + [ctypes.POINTER(ci)] * 5
         L.kg_junction_tile_of.argtypes = [ci, ci, ctypes.POINTER(ci), ctypes.POINTER(ci)]
         L.kg_gpool_tile_of.argtypes = [ci, ci, ci, ci] + [ctypes.POINTER(ci)] * 4
@@ -265,6 +267,17 @@ def conv_geometry(ks: int, ic: int, oc: int, split: bool, pixels: int) -> dict:
     g = ConvGeometry()
     _check(lib().kg_conv_geometry(ks, ic, oc, int(split), pixels, ctypes.byref(g)))
     return {f: getattr(g, f) for f, _ in ConvGeometry._fields_}
+
+
+SMALL_CONV3X3, SMALL_JUNCTION = 0, 1
+
+
+def small_tile_of(kernel: int, ic: int, oc: int, pixels: int, workgroup: int):
+    """(workgroups, tile rows, tile columns, pixel tile of `workgroup`, its column tile) of a 16-bit launch over few pixels;
+    0 workgroups where the large tiles run."""
+    out = [ctypes.c_int() for _ in range(5)]
+    _check(lib().kg_small_tile_of(kernel, ic, oc, pixels, workgroup, *[ctypes.byref(o) for o in out]))
+    return tuple(o.value for o in out)
 
 
 def float_tile_of(ks: int, rows: int, cols: int, k: int, workgroup: int):

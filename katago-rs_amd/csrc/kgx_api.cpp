@@ -625,11 +625,35 @@ int kg_float_tile_of(int ks, int rows, int cols, int k, int workgroup, int* grid
     if (!grid || !tile_rows || !tile_cols || !row_tile || !col_tile) throw std::runtime_error("null output");
     if ((ks != 1 && ks != 3) || rows < 1 || cols < 1 || k < 1 || (ks == 1 && !kgx::gemm_split_fits(cols, k, 0)))
       throw std::runtime_error("bad product shape");
-    const kgx::SplitGeometry g = kgx::split_geometry(ks, rows, cols, k, std::max(workgroup, 0), *row_tile, *col_tile);
+    const kgx::LaunchGeometry g = kgx::split_geometry(ks, rows, cols, k, std::max(workgroup, 0), *row_tile, *col_tile);
     *grid = g.grid;
     *tile_rows = g.tile_rows;
     *tile_cols = g.tile_cols;
     if (workgroup < 0 || workgroup >= g.grid) throw std::runtime_error("workgroup out of range");
+  });
+}
+
+int kg_small_tile_of(int kernel, int ic, int oc, int pixels, int workgroup, int* grid, int* tile_rows, int* tile_cols,
+                     int* pixel_tile, int* col_tile) {
+  return guarded([&] {
+    if (!grid || !tile_rows || !tile_cols || !pixel_tile || !col_tile) throw std::runtime_error("null output");
+    if (kernel != KG_SMALL_CONV3X3 && kernel != KG_SMALL_JUNCTION) throw std::runtime_error("unknown kernel");
+    if (pixels < 1 || (kernel == KG_SMALL_CONV3X3 && (ic < 1 || oc < 1))) throw std::runtime_error("bad convolution shape");
+    kgx::LaunchGeometry g;
+    *pixel_tile = *col_tile = 0;
+    if (kernel == KG_SMALL_CONV3X3) {
+      if (const int mb = kgx::conv_igemm_small_mb(3, ic, oc, pixels))
+        g = kgx::conv_small_geometry(mb, oc, pixels, std::max(workgroup, 0), *pixel_tile, *col_tile);
+    } else if (kgx::junction_tile_pixels(pixels) < 48) {
+      g.tile_rows = kgx::junction_tile_pixels(pixels);
+      g.tile_cols = kgx::kJunctionInner;
+      g.grid = (pixels + g.tile_rows - 1) / g.tile_rows;
+      *pixel_tile = std::max(workgroup, 0);
+    }
+    *grid = g.grid;
+    *tile_rows = g.tile_rows;
+    *tile_cols = g.tile_cols;
+    if (g.grid && (workgroup < 0 || workgroup >= g.grid)) throw std::runtime_error("workgroup out of range");
   });
 }
 

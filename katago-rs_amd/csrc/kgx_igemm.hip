@@ -827,6 +827,10 @@ void conv_igemm_pack_weights(int ks, const float* w, int oc, int ic, std::vector
       }
 }
 
+int conv_igemm_small_mb(int ks, int ic, int oc, int M) {
+  return igemm_kind(ks, ic, oc, false) == IG3_48 ? conv_small_mb(ks, ic, conv_igemm_icp(ks, ic, oc, false), oc, M) : 0;
+}
+
 void launch_conv_igemm(int prec, int ks, const void* x, int ldx, int IC, const void* w, int icp, int OC,
                        const ConvOut& o, int B, hipStream_t s, const void* x_lo) {
   if (prec != PREC_F16 && prec != PREC_BF16) throw std::runtime_error("conv_igemm: 16-bit operands only");
@@ -847,8 +851,8 @@ void launch_conv_igemm(int prec, int ks, const void* x, int ldx, int IC, const v
       throw std::runtime_error("conv_igemm: unsupported pooling partials");
   }
   const int M = B * HW, kind = igemm_kind(ks, IC, OC, split);
-  if (kind == IG3_48) {
-    if (const int mb = conv_small_mb(ks, IC, icp, OC, M)) {
+  if (!split) {
+    if (const int mb = conv_igemm_small_mb(ks, IC, OC, M)) {
       launch_conv_small(prec, mb, x, ldx, w, icp, OC, o, M, Ig3::BN, s);
       KGX_CHECK_LAUNCH();
       return;

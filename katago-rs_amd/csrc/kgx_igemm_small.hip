@@ -27,6 +27,12 @@ constexpr int SLD = SN + 4;          // the epilogue's float tile row stride
 
 __host__ __device__ constexpr int small_rows(int mb) { return 64 * mb + 2 * SHALO; }  // staged pixel rows, multiple of 8
 
+// Pixel tile mt, column tile nt of workgroup g of ntl column tiles.
+__host__ __device__ inline void small_tile_of(int g, int ntl, int& mt, int& nt) {
+  mt = g / ntl;
+  nt = g - mt * ntl;
+}
+
 // SC: as igemm_kernel's (kgx_igemm.hip).
 template <typename T, int MB, int SC>
 __global__ __launch_bounds__(SNT, 2) void conv_small_kernel(const T* __restrict__ X, int ldx, const T* __restrict__ W,
@@ -38,7 +44,8 @@ __global__ __launch_bounds__(SNT, 2) void conv_small_kernel(const T* __restrict_
   __shared__ __align__(1024) char smem[ZERO + 128];
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int grp = wv >> 2, wm = wv & 3, r16 = lane & 15, g4 = lane >> 4;
-  const int mt = blockIdx.x / ntl, nt = blockIdx.x - mt * ntl;
+  int mt, nt;
+  small_tile_of(blockIdx.x, ntl, mt, nt);
   const int m0 = mt * BM, n0 = nt * SN, nk = icp / SK;
   char* const Ab = smem + SSTAGES * WST;
 
@@ -168,7 +175,7 @@ __global__ __launch_bounds__(SNT, 2) void conv_small_kernel(const T* __restrict_
 }  // namespace
 
 // MB of the launch over M pixels and OC outputs: the smallest tile whose workgroups all run at once (one per CU:
-// its stages take 97-142 KB of LDS), 0 where none does (more than 4032 pixels at 192 outputs, batch 11) or the
+// its stages take 95 to 145 KB of LDS), 0 where none does (more than 4032 pixels at 192 outputs, batch 11) or the
 // channels do not fit the kernel.
 int conv_small_mb(int ks, int ic, int icp, int oc, int M) {
   if (ks != 3 || ic != icp || icp > SSTAGES * SK || M < 1) return 0;
@@ -178,10 +185,21 @@ int conv_small_mb(int ks, int ic, int icp, int oc, int M) {
   return 0;
 }
 
+static int small_grid(int mb, int OC, int M) { return (M + 64 * mb - 1) / (64 * mb) * ((OC + SN - 1) / SN); }
+
+LaunchGeometry conv_small_geometry(int mb, int oc, int M, int g, int& mt, int& nt) {
+  small_tile_of(g, (oc + SN - 1) / SN, mt, nt);
+  LaunchGeometry r;
+  r.grid = small_grid(mb, oc, M);
+  r.tile_rows = 64 * mb;
+  r.tile_cols = SN;
+  return r;
+}
+
 template <typename T, int MB>
 static void small_launch(const void* x, int ldx, const void* w, int icp, int OC, const ConvOut& o, int M, int pbn,
                          hipStream_t s) {
-  const int ntl = (OC + SN - 1) / SN, grid = (M + 64 * MB - 1) / (64 * MB) * ntl;
+  const int ntl = (OC + SN - 1) / SN, grid = small_grid(MB, OC, M);
   auto go = [&](auto kernel) {
     launch_k(kernel, grid, SNT, 0, s, (const T*)x, ldx, (const T*)w, icp, OC, M, ntl, pbn, o);
   };

@@ -465,6 +465,8 @@ int junction_tile_of(int g) { return junction_tile(g); }
 // 16-row blocks per workgroup over M pixels: the fewest whose workgroups all run at once (one per CU).
 int junction_blocks(int M) { return M <= 256 * junction_rows(1) ? 1 : M <= 256 * junction_rows(2) ? 2 : 3; }
 
+int junction_tile_pixels(int M) { return junction_rows(junction_blocks(M)); }
+
 int junction_grid(int M) {
   const int regions = (M + 4 * JR48 - 1) / (4 * JR48);
   return 32 * ((regions + 7) / 8);

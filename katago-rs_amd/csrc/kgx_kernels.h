@@ -173,6 +173,10 @@ const char* conv_igemm_class(int ks, int ic, int oc, bool split = false);
 // per tile (BN) when its kernel computes pooling partials (3x3 with 64-channel column tiles, 192 pixels), else 0.
 int conv_igemm_tile_rows(int ks, int ic, int oc, bool split = false);
 int conv_igemm_pool_cols(int ks, int ic, int oc);
+// A launch's workgroups and tile.
+struct LaunchGeometry {
+  int grid = 0, tile_rows = 0, tile_cols = 0;
+};
 // The launch geometry of the convolution of these shapes over M pixels on the large tiles (launch_conv_igemm runs few
 // pixels on conv_small_mb's), and the index maps its kernel uses (the
 // same functions): workgroup -> (pixel tile, column tile), -1 for a workgroup that exits at once; with the weights
@@ -197,6 +201,10 @@ void launch_conv_igemm(int prec, int ks, const void* x, int ldx, int IC, const v
 // results as launch_conv_igemm's 48-column 3x3, on tiles of 64 mb pixels x 16 channels; conv_small_mb is 0 where that
 // one runs.
 int conv_small_mb(int ks, int ic, int icp, int oc, int M);
+// conv_small_mb of the convolution that launch_conv_igemm runs (0: on the large tiles), and the launch's grid, tile and the
+// tiles of workgroup g.
+int conv_igemm_small_mb(int ks, int ic, int oc, int M);
+LaunchGeometry conv_small_geometry(int mb, int oc, int M, int g, int& mt, int& nt);
 void launch_conv_small(int prec, int mb, const void* x, int ldx, const void* w, int icp, int OC, const ConvOut& o, int M,
                        int pbn, hipStream_t s);
 // Float 3x3 convolution on bf16 matrix cores (kgx_split.hip): x float NHWC rows of ldx (IC % 8 == 0), OC % 4 == 0, w the
@@ -206,10 +214,7 @@ void launch_conv_split_pack(const float* w, int oc, int ic, void* out, hipStream
 void launch_conv_split(const float* x, int ldx, int IC, const void* w, int OC, const ConvOut& o, int B, hipStream_t s);
 // The grid and tile that a float 3x3 convolution (ks 3: M pixels, K -> N channels) or GEMM (ks 1: M x N over K) of kgx_split.hip
 // runs on, and the tiles of workgroup g (-1 when it exits at once).
-struct SplitGeometry {
-  int grid = 0, tile_rows = 0, tile_cols = 0;
-};
-SplitGeometry split_geometry(int ks, int M, int N, int K, int g, int& row_tile, int& col_tile);
+LaunchGeometry split_geometry(int ks, int M, int N, int K, int g, int& row_tile, int& col_tile);
 // The value a float becomes as a compute-type operand (round to nearest even), as a float.
 float conv_round_operand(float v, int prec);
 
@@ -225,8 +230,10 @@ constexpr int kJunctionInner = 192, kJunctionOuter = 384, kJunctionHead = 96;
 void junction_pack_weights(const float* w_exit, const float* w_entry, int entry_oc, int prec, std::vector<float>& out);
 void launch_junction(int prec, const void* x, const void* x_lo, int ldx, const void* w, const ConvOut& exit_o,
                      const ConvOut& entry_o, int entry_oc, int B, hipStream_t s);
-// The 48-pixel launch's grid over M pixels (above 8192; fewer take smaller tiles), and the tile workgroup g computes (tiles past M exit at once).
+// The 48-pixel launch's grid over M pixels (above 8192; fewer take smaller tiles), and the tile workgroup g computes (tiles
+// past M exit at once); the pixels per workgroup that a launch over M pixels takes (16 and 32: workgroup g tile g).
 int junction_grid(int M);
+int junction_tile_pixels(int M);
 // The stem junction: the network's stem, a 3x3 convolution of the packed input rows (ldx <= 32 channels, one 16-bit
 // plane) into the trunk with its row bias (eo: y stored, colbias, the emission of the entry's activation), and the
 // first nested block's entry 1x1 (384 -> 192, split operands), in one launch over junction_grid(M) workgroups.

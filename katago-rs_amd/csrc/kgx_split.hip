@@ -771,8 +771,8 @@ int gemm_split_rows(int M, int N, int K) {
   return t96 <= t32 ? 96 : 32;
 }
 
-SplitGeometry split_geometry(int ks, int M, int N, int K, int g, int& row_tile, int& col_tile) {
-  SplitGeometry r;
+LaunchGeometry split_geometry(int ks, int M, int N, int K, int g, int& row_tile, int& col_tile) {
+  LaunchGeometry r;
   if (ks == 3) {
     const int(&t)[2] = conv_split_tile(M, N);
     r.tile_rows = 16 * t[0];

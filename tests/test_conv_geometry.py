@@ -192,3 +192,29 @@ def test_float_tile_rule_counts_the_busiest_xcd(kgx, ks, rows, cols, k):
     grid = kgx.float_tile_of(ks, rows, cols, k, 0)[0]
     load = collections.Counter(wg % 8 for wg in range(grid) if kgx.float_tile_of(ks, rows, cols, k, wg)[3] >= 0)
     assert max(load.values()) <= 32, load
+
+
+# The 16-bit 3x3 shapes with a small launch, and the batches from which the large tiles run.
+@pytest.mark.parametrize("ic,oc,large_from", [(192, 192, 12), (128, 128, 18), (64, 72, 28), (192, 256, 1), (22, 384, 1)])
+def test_small_convolution_tiles_are_computed_once(kgx, ic, oc, large_from):
+    for b in range(1, large_from + 2):
+        pixels = b * 361
+        grid, tr, tc = kgx.small_tile_of(kgx.SMALL_CONV3X3, ic, oc, pixels, 0)[:3]
+        assert (grid > 0) == (b < large_from), b
+        if not grid:
+            continue
+        assert grid <= 256  # one round
+        seen = collections.Counter(kgx.small_tile_of(kgx.SMALL_CONV3X3, ic, oc, pixels, g)[3:] for g in range(grid))
+        assert set(seen) == {(m, n) for m in range(-(-pixels // tr)) for n in range(-(-oc // tc))}, b
+        assert all(v == 1 for v in seen.values())
+        with pytest.raises(kgx.KgError, match="workgroup out of range"):
+            kgx.small_tile_of(kgx.SMALL_CONV3X3, ic, oc, pixels, grid)
+
+
+def test_small_junction_tiles_are_computed_once(kgx):
+    for b in range(1, 25):
+        grid, tr = kgx.small_tile_of(kgx.SMALL_JUNCTION, 0, 0, b * 361, 0)[:2]
+        assert (grid > 0) == (b <= 22) and tr == (16 if b <= 11 else 32 if b <= 22 else 0), b
+        tiles = [kgx.small_tile_of(kgx.SMALL_JUNCTION, 0, 0, b * 361, g)[3] for g in range(grid)]
+        assert tiles == list(range(-(-b * 361 // tr) if tr else 0))
+        assert grid <= 256
