@@ -37,6 +37,8 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 PEAK_TFLOPS = {"f16": 2500.0, "bf16": 2500.0, "f32": 157.3}  # MI355X dense MFMA
+# A float product on three bf16 planes per operand is six bf16 products.
+PEAK_F32_SPLIT_TFLOPS = PEAK_TFLOPS["bf16"] / 6
 PEAK_HBM_GBS = 8000.0
 # The headline metric's name for the default workload; other workloads are named the same way.
 HEADLINE = "evals/s b18c384nbt fp16 batch 32 on 1 MI355X; MFMA util % + HBM GB/s %"
@@ -46,6 +48,11 @@ TRACE_FILE = os.path.join(ROOT, "profiles", "kernel_trace.json")
 PUBLISHED_FLEX = {"b10c128 batch 8": 33.0, "b18c384nbt batch 8": 2.5}
 # The reference's published ROCm f32 throughput of b10c128 at batch 8 on an RX 6800 XT (README.md:85-86), evals/s.
 PUBLISHED_B10C128_F32_B8 = 2617.0
+
+
+def class_peak(precision, kernel_class):
+    """The TFLOP/s ceiling of a kernel class: float handles' `_split` classes run on the bf16 units."""
+    return PEAK_F32_SPLIT_TFLOPS if precision == "f32" and kernel_class.endswith("_split") else PEAK_TFLOPS[precision]
 
 
 def copy_probe(mb):
@@ -301,7 +308,7 @@ def main():
         # latency-bound kernels reach neither, and the 1x1 convolutions' bound is the higher one.
         if v["flops"] > 0:
             c["tflops"] = v["flops"] / (v["ms"] * 1e-3) / 1e12
-            c["mfma_frac"] = c["tflops"] / PEAK_TFLOPS[args.precision]
+            c["mfma_frac"] = c["tflops"] / class_peak(args.precision, k)
         if v["bytes"] > 0:
             c["gbs"] = v["bytes"] / (v["ms"] * 1e-3) / 1e9
             c["hbm_frac"] = c["gbs"] / PEAK_HBM_GBS
@@ -311,7 +318,7 @@ def main():
     per_launch_ms = dv["ms"] / max(dv["launches"], 1)
     if dv["flops"] > 0:
         achieved = dv["flops"] / max(dv["launches"], 1) / (per_launch_ms * 1e-3) / 1e12
-        peak = PEAK_TFLOPS[args.precision]
+        peak = class_peak(args.precision, dname)
         roof = {"bound": "mfma", "kernel": dname, "achieved": achieved, "peak": peak, "unit": "TFLOP/s",
                 "frac": achieved / peak, "traffic": None,
                 "work_per_launch": dv["flops"] / max(dv["launches"], 1), "avg_launch_us": per_launch_ms * 1e3}

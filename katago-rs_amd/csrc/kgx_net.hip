@@ -133,6 +133,16 @@ const void* Net::upload_t(const std::vector<float>& v) {
   return d;
 }
 
+// The profile class of a GEMM of class `cls` on three-plane operands, which run against another peak.
+static const char* split3_class(const char* cls) {
+  const std::string c = cls;
+  if (c == "token_gemm_qkv") return "token_gemm_qkv_split";
+  if (c == "token_gemm_out") return "token_gemm_out_split";
+  if (c == "token_gemm_ffn1") return "token_gemm_ffn1_split";
+  if (c == "token_gemm_ffn2") return "token_gemm_ffn2_split";
+  return "gemm_1x1_split";
+}
+
 // Whether a GEMM runs as a three-plane product of float operands, and its weights' upload (B^T rows [N][K]).
 bool Net::gemm_split(int N, int K, int dq) const { return conv_mode_ == CONV_SPLIT && gemm_split_fits(N, K, dq); }
 
@@ -465,10 +475,10 @@ std::shared_ptr<ConvOut> Net::emit_conv(const ConvDesc& c, const void* x, int ld
       g.split3 = split3;
       launch_gemm(prec, g, s);
     };
-    gm.cls = "gemm_1x1";
+    gm.cls = split3 ? split3_class("gemm_1x1") : "gemm_1x1";
     gm.flops_row = 2.0 * HW * ic * oc;
     gm.bytes_row = in_bytes + out_bytes;
-    gm.bytes_fixed = (double)ic * oc * ts;
+    gm.bytes_fixed = (double)ic * oc * (split3 ? 6 : ts);
     gm.out = out;
     gm.out_c = oc;
     ops_.push_back(gm);
@@ -512,13 +522,13 @@ std::shared_ptr<ConvOut> Net::emit_token_gemm(const void* A, int lda, const void
     g.yt_act = yt_act;
     launch_gemm(prec, g, s);
   };
-  op.cls = cls;
+  op.cls = split3 ? split3_class(cls) : cls;
   const double ts = (double)tsize();
   op.flops_row = 2.0 * HW * K * N;
   op.bytes_row = (double)HW * K * ts +
                  (double)HW * N * ((o.y ? 4.0 : 0.0) * (o.accumulate ? 2 : 1) + (o.yt ? (glu ? ts / 2 : ts) : 0.0) +
                                    (o.emit.scale ? ts : 0.0));
-  op.bytes_fixed = (double)K * N * ts;
+  op.bytes_fixed = (double)K * N * (split3 ? 6 : ts);
   op.out = out;
   op.out_c = N;
   ops_.push_back(op);

@@ -245,6 +245,12 @@ def test_copy_outputs_sentinels_follow_every_reference_branch(kgx):
         kgx.copy_outputs(spec.sentinel_row(1, 6)[None], 1, 6, 9, 8, 0.0)
 
 
+def test_bench_prices_float_split_classes_against_the_bf16_units():
+    import bench
+    assert bench.class_peak("f32", "conv3x3_split") == bench.class_peak("f32", "token_gemm_ffn1_split") == 2500.0 / 6
+    assert bench.class_peak("f32", "gemm_1x1") == 157.3 and bench.class_peak("f16", "conv3x3") == 2500.0
+
+
 def test_output_rows_own_their_memory(kgx):
     """The policy and ownership of a row belong to it: keeping one row (a cache of evaluations) keeps no other's, and
     writing to it changes no other's."""
