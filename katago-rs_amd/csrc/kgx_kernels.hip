@@ -1104,13 +1104,14 @@ void launch_tip_rms(const float* x, int C, const float* gamma, const float* beta
 //   D / 16 floats per lane at dims (D / 16) l16 .., which makes output row i of tile dt dim (D / 16) i + dt.
 // The four waves' maxima, sums and outputs meet in LDS. Bound: the chain of one wave (its loads and 192 QT MFMAs of 32
 // cycles) at small batches, the matrix cores' float rate (157 TFLOP/s) at large ones. One thread per query on the
-// vector units, keys staged in LDS, before this: 315 -> 18.6 us at 3 rows of 6 heads of 64 dims, 328 -> 41 us at 10 rows
-// of 8 heads (65 TFLOP/s), 76 TFLOP/s at 24 rows of 6.
+// vector units, keys staged in LDS, before this: 315 -> 17.9 us at 3 rows of 6 heads of 64 dims, 326 -> 36.8 us at 10 rows
+// of 8 heads (73 TFLOP/s).
 constexpr int ATF_NW = 4, ATF_KT = (HW + 15) / 16, ATF_WT = (ATF_KT + ATF_NW - 1) / ATF_NW;  // key tiles, per wave
 // Up to this many (row, head) pairs a workgroup takes 16 queries, beyond it 32 (half the reads of K and V per query):
-// 10.8 against 13.8 us at 6 heads of 64 dims (1 row of b10c384h6), 18.6 against 19.1 at 18, but 23.4 against 20.6 at 40
-// (5 rows of b10c512h8), 45.3 against 41.2 at 80 and 123 against 114 at 256.
-constexpr int ATF_NARROW_HEADS = 20;
+// 11.1 against 14.1 us at 6 heads of 64 dims (1 row of b10c384h6), 17.9 against 19.3 at 18 and 17.8 against 19.2 at 24 (3 rows
+// of b10c512h8; the wide blocks are past one round of CUs there), but 23.0 against 20.7 at 40, 40.1 against 36.8 at 80
+// and 107 against 95 at 256.
+constexpr int ATF_NARROW_HEADS = 24;
 
 // The W floats at byte offset off of [base, base + nbytes), 0 past the range (a buffer load: no branch, no 64-bit address).
 template <int W>

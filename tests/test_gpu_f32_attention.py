@@ -1,5 +1,5 @@
 """Attention of float handles (attn_f32_kernel): every head dim, shared key/value heads, learnable and no rotation, on
-ragged boards, against the oracle; and rows that do not depend on the batch across the two query-block widths (up to 20
+ragged boards, against the oracle; and rows that do not depend on the batch across the two query-block widths (up to 24
 (row, head) pairs take 16 queries per workgroup, more take 32)."""
 import numpy as np
 import pytest
@@ -14,7 +14,7 @@ def test_float_attention_matches_oracle_at_both_widths(kgx, synth, oracle, heads
                                               ("attn", heads, kv, dim, dim, rope)],
                       p1_c=16, g1_c=16, v1_c=16, v2_c=24, qk_gain=2.0)
     mb = synth.write_model(arch, 17)
-    n = 20 // heads + 2  # the whole batch takes the wide blocks, up to 20 // heads rows the narrow ones
+    n = 20 // heads + 2  # the whole batch takes the wide blocks, up to 24 // heads rows the narrow ones
     sp, gl, _ = synth.make_inputs(n, 23, board_sizes=[19, 9, 13, 2])
     net = kgx.Net(mb)
     h = kgx.Handle(net, n, "f32")
@@ -46,7 +46,7 @@ def test_float_attention_scores_far_below_zero(kgx, synth, oracle):
     put(t["stem_mm"], np.zeros_like(t["stem_mm"]))
     put(b["q"], np.eye(64, dtype=np.float32) * np.float32(1e16))
     put(b["k"], np.eye(64, dtype=np.float32) * np.float32(-1e16))
-    n = 24  # both query-block widths
+    n = 25  # both query-block widths
     sp, gl, _ = synth.make_inputs(n, 3)
     sp = sp.reshape(n, 22, 361).copy()
     sp[:, 1] = 0.0
