@@ -1,8 +1,11 @@
-// Float 3x3 convolutions and GEMMs on the bf16 matrix cores. Every float operand is split into three bf16 planes, x = h + m + l
-// (each the rounding of what the planes before it leave: 24 significant bits, float's exponent range), and a product
-// is taken as l h + m m + m h + h l + h m + h h with float accumulation; the terms left out are below 2^-26 of the
-// product. Six v_mfma_f32_16x16x32_bf16 take 96 cycles where v_mfma_f32_16x16x4_f32 takes 256 for the same products,
-// and the direct sum has neither the transforms' traffic of Winograd F(4x4,3x3) nor its loss of accuracy.
+// Float 3x3 convolutions and GEMMs on the bf16 matrix cores. Every float operand is split into three bf16 planes,
+// x = h + m + l (each the rounding of what the planes before it leave: 24 significant bits, float's exponent range), and a
+// product is taken as l h + m m + m h + h l + h m + h h with float accumulation. The terms left out (m l + l m + l l) are
+// at most 2^-23 of the product, where a float product rounds by 2^-24: in sums of 32 terms and more the sums' rounding
+// covers them (the error against 64 bits fell in every network measured); a sum that one product carries may be off by
+// 1.0e-7 of it instead of 6e-8. Six v_mfma_f32_16x16x32_bf16 take 96 cycles where v_mfma_f32_16x16x4_f32 takes 256 for
+// the same products, and the direct sum has neither the transforms' traffic of Winograd F(4x4,3x3) nor its loss of
+// accuracy.
 //
 // A workgroup computes 16 MB pixels x 16 NB channels. Per chunk of 64 input channels it stages the pixel rows (tile and
 // a halo of 20, as kgx_igemm.hip) in LDS as three planes, split in registers on the way, in two buffers with one
@@ -12,14 +15,14 @@
 // never passes through LDS. The pairs' sums are added through LDS in order, which the tile's size does not change: a
 // row's results do not depend on the batch.
 //
-// 192 -> 192 channels at 16 boards (96 x 48 tiles, 244 workgroups): 23.5 us, against 53 us of input transform, 36 point
-// GEMMs and output transform (F(4x4,3x3)); 128 -> 128 at 8 boards (48 x 32): 9.1 against 37 us. The MFMAs are 12 us of
+// 192 -> 192 channels at 16 boards (96 x 48 tiles, 244 workgroups): 23.7-24.6 us, against 53 us of input transform, 36 point
+// GEMMs and output transform (F(4x4,3x3)); 128 -> 128 at 8 boards (48 x 32): 9.3-9.6 against 37 us. The MFMAs are 12 us of
 // the first; splitting the operands costs 2.5 us of VALU time, the first stage and the epilogue 4.
 // An activation that is infinite, or rounds to infinity as a bf16 (from 3.3962e38), has no planes (inf - inf). A GEMM's
 // sum that comes out infinite or NaN is therefore taken again on the float matrix unit (float_sums), which keeps the
 // infinities and the top of the range; a 3x3 convolution gives NaN there, as the Winograd transforms do. Weights keep their
-// value at the top of the range (their first plane is cut, not rounded, where it would overflow). Below 2^-110 (7.7e-34)
-// the last planes fall under the smallest bf16, and an operand keeps fewer bits.
+// value at the top of the range (their first plane is cut, not rounded, where it would overflow). Below 2^-103 (1e-31) the
+// last planes fall under the smallest normal bf16, and an operand keeps fewer bits.
 #include "kgx_gemm_epi.h"
 
 #include <cfloat>
@@ -329,9 +332,9 @@ __global__ __launch_bounds__(PNT, 1) void conv3_split_kernel(const float* __rest
 // its serial K loop sets the time) runs a quarter of the steps one after the other. The pairs' sums are added in
 // order, whatever the tile. The waves of a pair split the rows (MB = 6) or the columns (MB = 2).
 // Against the float matrix unit's 64 x 64 tiles (one 16-channel stage after the other): N = 384 over K = 384 and 1536 at
-// 1083 rows 32.7 -> 12.7 us on average, K = 384 into 1536 columns 28.3 -> 21.5; against its 128 x 128 tiles at 3610
-// rows, where both operands' reads from L2 bound it (about 64 bytes a cycle and CU), 149 -> 140 and 76 -> 59 us
-// (gemm_split_lds_kernel takes those).
+// 1083 rows 33.0 -> 12.8 us on average; N = 512 over K = 512 and 2048 at 3610 rows 64.2 -> 52.9 on average (80.0 for K = 2048
+// here, 25.9 for K = 512 in gemm_split_lds_kernel). Where the rounds are many, both operands' reads from L2 bound it (about
+// 64 bytes a cycle and CU): gemm_split_lds_kernel takes those.
 template <int MB, int EPI>
 __global__ __launch_bounds__(PNT, MB == 2 ? 4 : 2) void gemm_split_kernel(const float* __restrict__ A, const bf16* __restrict__ W, int lda,
                                                             int M, int N, int K, int ntl, GemmArgs g) {

@@ -1,6 +1,6 @@
 """The allocation-free forward pass (kg_run_static, workspace in the library's static device array) against the
 ordinary one (kg_run), through the C ABI: bit-identical rows on two calls in a row, the second with fewer rows, on
-nets covering the implicit-GEMM and split-operand convolutions, the Winograd path (float) and transformer blocks;
+nets covering the implicit-GEMM and split-operand convolutions, the float paths (the direct sum, and Winograd in the stem) and transformer blocks;
 and the rejection of a batch beyond the static scratch's capacity."""
 
 import ctypes
